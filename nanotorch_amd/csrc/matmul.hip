@@ -11,16 +11,19 @@
 //               or B = W^T of a row-major W).  Stored in LDS as [mn][k].
 //   layout MN : the m (or n) index is unit-stride (A = X^T of a row-major
 //               X, or B row-major).  Stored in LDS as [k][mn].
-//   layout GEN: anything else (e.g. `[:, ::2]` views): scalar loads, stored
-//               as [mn][k].
+//   anything else (odd row lengths, `[:, ::2]` views): 4-byte loads along
+//               the axis with the smaller stride, stored either way.
 //
-// Workgroup tile 128x128, k-tile 32, 256 threads = 4 waves in a 2x2 grid,
-// each wave owns a 64x64 block = 2x2 MFMA 32x32 blocks (64 accumulator
-// registers per lane).  Global loads for k-tile t+1 are issued before the
-// MFMAs of tile t; LDS is double buffered so one barrier per k-tile
-// suffices.  Workgroups are numbered so that consecutive tiles of a group of
-// 8 tile-rows land on the same XCD (gfx950 dispatches workgroups round-robin
-// over its 8 XCDs, each with its own L2).
+// Workgroup tiles of 128x128, 64x64, 32x128 and 128x32 with a 32-deep k-tile
+// (mm_f32_tile_kernel, 256 threads = 4 waves), and of 256x256 for large
+// products whose sizes fit (mm_f32_mfma_wide_kernel, 8 waves).  Operands go
+// from global memory straight into LDS (gfx950's direct loads, 16 bytes per
+// lane where the layout allows and 4 bytes otherwise); LDS is double
+// buffered and the loads of k-tile t+1 are in flight under the MFMAs of tile
+// t, with one barrier per k-tile.  The tile shape and a split of K follow
+// the product's size (choose_tile).  Workgroups are numbered so that
+// consecutive tiles of a group of 8 tile-rows land on the same XCD (gfx950
+// dispatches workgroups round-robin over its 8 XCDs, each with its own L2).
 //
 // MFMA k assignment: in MFMA step kk (0..15) of a k-tile, the lanes of wave
 // half h (lane / 32) supply k = h*16 + kk, for A and B alike, so each lane's
@@ -30,40 +33,22 @@
 // bound).  Accumulate mode adds C_old after the full dot product: one
 // rounding, like the reference's `x._grad += grad`.
 //
-// When both operands are in a vector layout and K is a multiple of 32, the
-// operands skip the register round trip: mm_f32_mfma_dl_kernel stages them
-// with gfx950's direct global-to-LDS loads (same tiles, same MFMA schedule).
-// Large products (M, N multiples of 256, K of 64, a 256x256 tile per CU)
-// use mm_f32_mfma_wide_kernel: 256x256 tiles, 8 waves of 128x64.
-//
 // Other dtypes (fp64, int32, int64) use a tiled SIMT kernel that accumulates
 // in k order exactly like the reference's CPU loop (matmul.cu:33-45).
 #include <algorithm>
+#include <limits>
 
-#include "nt_internal.h"
+#include "ew_engine.h"
 
 namespace nt {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
-// Largest split of K for a single product with fewer wide tiles than CUs.
-#ifndef NT_MM_SPLITK_MAX
-#define NT_MM_SPLITK_MAX 8
-#endif
-// The split-K sum kernel is instantiated for 2, 4 and 8 slices only.
-static_assert(NT_MM_SPLITK_MAX == 1 || NT_MM_SPLITK_MAX == 2 ||
-                  NT_MM_SPLITK_MAX == 4 || NT_MM_SPLITK_MAX == 8,
-              "NT_MM_SPLITK_MAX must be 1, 2, 4 or 8");
-
-constexpr int MM_BM = 128, MM_BN = 128, MM_BK = 32, MM_THREADS = 256;
-constexpr int MM_KPAD = MM_BK + 4;  // [mn][k] row length (floats)
-constexpr int MM_MNPAD = MM_BM + 4; // [k][mn] row length (floats)
-constexpr int MM_REGION = (MM_BM * MM_KPAD > MM_BK * MM_MNPAD)
-                              ? MM_BM * MM_KPAD
-                              : MM_BK * MM_MNPAD; // floats per operand stage
+constexpr int MM_BK = 32, MM_THREADS = 256;
 constexpr int MM_MAX_BATCH = NT_MAX_DIMS - 2;
 
-enum { LAY_K = 0, LAY_MN = 1, LAY_GEN = 2 };
+// Unit-stride axis of an operand of the wide kernel.
+enum { LAY_K = 0, LAY_MN = 1 };
 
 struct MMArgs {
   const float *A;
@@ -75,11 +60,12 @@ struct MMArgs {
   int64_t bshape[MM_MAX_BATCH];
   int64_t bsA[MM_MAX_BATCH], bsB[MM_MAX_BATCH], bsC[MM_MAX_BATCH];
   int64_t tiles_m, tiles_n;
+  uint32_t nbatch;
   int accumulate;
-  // Wide kernel, split over K: blockIdx.y = s takes k in [s kslice,
-  // (s + 1) kslice) and writes its raw sum to part + s M N ([M][N]
-  // contiguous); mm_splitk_sum_kernel adds the slices.  part == nullptr: no
-  // split (kslice == K), results go to C.
+  // Split over K: slice s takes k in [s kslice, (s + 1) kslice) and writes
+  // its raw sum to part + s nbatch M N (every batch [M][N] contiguous);
+  // mm_splitk_sum_kernel adds the slices.  part == nullptr: no split (one
+  // slice, kslice >= K), results go to C.
   int64_t kslice;
   float *part;
   // Optional bias added to every output row in the epilogue, C = fl(acc) +
@@ -89,118 +75,46 @@ struct MMArgs {
   int64_t sBias;
 };
 
-// Operand tile loader: global -> registers -> LDS.  ROWS x MM_BK tile of
-// the operand in (mn, k) coordinates, where mn is m for A and n for B.
-// s_mn / s_k are the element strides of the mn and k indices.
-template <int LAY> struct TileLoad {
-  float4 r[4];
-  __device__ __forceinline__ void load(const float *p, int64_t mn0, int64_t k0,
-                                       int64_t MN, int64_t K, int64_t s_mn,
-                                       int64_t s_k, int t) {
-    if constexpr (LAY == LAY_K) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int64_t mn = mn0 + (t >> 3) + 32 * i;
-        const int64_t k = k0 + (t & 7) * 4;
-        if (mn < MN && k < K)
-          r[i] = *reinterpret_cast<const float4 *>(p + mn * s_mn + k);
-        else
-          r[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-    } else if constexpr (LAY == LAY_MN) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int64_t k = k0 + (t >> 5) + 8 * i;
-        const int64_t mn = mn0 + (t & 31) * 4;
-        if (mn < MN && k < K)
-          r[i] = *reinterpret_cast<const float4 *>(p + mn + k * s_k);
-        else
-          r[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float v[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int flat = t + MM_THREADS * (4 * i + q); // 0..4095
-          const int64_t mn = mn0 + (flat >> 5);
-          const int64_t k = k0 + (flat & 31);
-          v[q] = (mn < MN && k < K) ? p[mn * s_mn + k * s_k] : 0.f;
-        }
-        r[i] = make_float4(v[0], v[1], v[2], v[3]);
-      }
-    }
-  }
-  __device__ __forceinline__ void store(float *lds, int t) const {
-    if constexpr (LAY == LAY_K) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int mn = (t >> 3) + 32 * i, k = (t & 7) * 4;
-        *reinterpret_cast<float4 *>(lds + mn * MM_KPAD + k) = r[i];
-      }
-    } else if constexpr (LAY == LAY_MN) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int k = (t >> 5) + 8 * i, mn = (t & 31) * 4;
-        *reinterpret_cast<float4 *>(lds + k * MM_MNPAD + mn) = r[i];
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float v[4] = {r[i].x, r[i].y, r[i].z, r[i].w};
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int flat = t + MM_THREADS * (4 * i + q);
-          lds[(flat >> 5) * MM_KPAD + (flat & 31)] = v[q];
-        }
-      }
-    }
-  }
-};
-
-// Fragment read: element (mn, k) of the staged tile.
-template <int LAY>
-__device__ __forceinline__ float frag(const float *lds, int mn, int k) {
-  if constexpr (LAY == LAY_MN)
-    return lds[k * MM_MNPAD + mn];
-  else
-    return lds[mn * MM_KPAD + k];
-}
-
-// Workgroup -> (batch, tile) with an XCD-contiguous numbering, then groups
-// of 8 tile-rows walked column by column; A, B, C advanced to the batch.
+// Workgroup -> (slice of K, batch, tile).
 struct TileCoord {
   int64_t m0, n0;
+  uint32_t slice, batch;
   const float *A, *B;
   float *C;
 };
 
-template <int BM = MM_BM, int BN = MM_BN>
+// The 1-D grid holds slices x batches x tiles.  Workgroup ids are dealt to
+// the 8 XCDs round-robin; renumbered so that each XCD gets one contiguous run
+// (of any grid size), tiles of a run walk groups of 8 tile-rows column by
+// column.  The grid is below 2^31 workgroups: 32-bit divisions.
+template <int BM, int BN>
 __device__ __forceinline__ TileCoord mm_tile_coord(const MMArgs &g) {
-  const int64_t per_batch = g.tiles_m * g.tiles_n;
-  int64_t bid = blockIdx.x;
-  const int64_t nblk = gridDim.x;
-  if (nblk % 8 == 0)
-    bid = (bid % 8) * (nblk / 8) + bid / 8;
-  const int64_t batch = bid / per_batch;
-  const int64_t tile = bid - batch * per_batch;
-  constexpr int64_t GROUP = 8;
-  const int64_t group = tile / (GROUP * g.tiles_n);
-  const int64_t first_m = group * GROUP;
-  const int64_t gsize = (g.tiles_m - first_m) < GROUP ? (g.tiles_m - first_m)
-                                                       : GROUP;
-  const int64_t in_group = tile - group * GROUP * g.tiles_n;
+  const uint32_t tm = uint32_t(g.tiles_m), tn = uint32_t(g.tiles_n);
+  const uint32_t per_batch = tm * tn;
+  const uint32_t nblk = gridDim.x, q8 = nblk / 8, r8 = nblk % 8;
+  const uint32_t xcd = blockIdx.x % 8;
+  const uint32_t bid = xcd * q8 + (xcd < r8 ? xcd : r8) + blockIdx.x / 8;
   TileCoord tc;
-  tc.m0 = (first_m + in_group % gsize) * BM;
-  tc.n0 = (in_group / gsize) * BN;
+  const uint32_t all = bid / per_batch; // slice * batches + batch
+  const uint32_t tile = bid - all * per_batch;
+  tc.slice = all / g.nbatch;
+  tc.batch = all - tc.slice * g.nbatch;
+  constexpr uint32_t GROUP = 8;
+  const uint32_t group = tile / (GROUP * tn);
+  const uint32_t first_m = group * GROUP;
+  const uint32_t gsize = tm - first_m < GROUP ? tm - first_m : GROUP;
+  const uint32_t in_group = tile - group * GROUP * tn;
+  const uint32_t col = in_group / gsize;
+  tc.m0 = int64_t(first_m + in_group - col * gsize) * BM;
+  tc.n0 = int64_t(col) * BN;
   tc.A = g.A;
   tc.B = g.B;
   tc.C = g.C;
-  int64_t rem = batch;
+  uint32_t rem = tc.batch;
   for (int d = g.nb - 1; d >= 0; --d) {
-    const int64_t q = rem / g.bshape[d];
-    const int64_t c = rem - q * g.bshape[d];
+    const uint32_t sz = uint32_t(g.bshape[d]);
+    const uint32_t q = rem / sz;
+    const int64_t c = rem - q * sz;
     rem = q;
     tc.A += c * g.bsA[d];
     tc.B += c * g.bsB[d];
@@ -209,111 +123,38 @@ __device__ __forceinline__ TileCoord mm_tile_coord(const MMArgs &g) {
   return tc;
 }
 
-// Lane holds column li of each 32x32 block, rows 8*(r/4) + 4*h + (r%4).
-__device__ __forceinline__ void mm_epilogue(const MMArgs &g, const TileCoord &tc,
-                                            const floatx16 (&acc)[2][2], int wm,
-                                            int wn, int h, int li) {
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int64_t col = tc.n0 + wn * 64 + j * 32 + li;
-      if (col >= g.N)
-        continue;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t row =
-            tc.m0 + wm * 64 + i * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
-        if (row < g.M) {
-          float *dst = tc.C + row * g.sCm + col * g.sCn;
-          const float v = acc[i][j][r];
-          *dst = g.accumulate ? (*dst + v) : (g.bias ? v + g.bias[col * g.sBias] : v);
-        }
-      }
-    }
-}
-
-template <int LA, int LB>
-__global__ __launch_bounds__(MM_THREADS, 2) void mm_f32_mfma_kernel(MMArgs g) {
-  __shared__ __align__(16) float lds[2][2][MM_REGION]; // [stage][A/B]
-  const int t = threadIdx.x;
-  const int lane = t & 63, wave = t >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int h = lane >> 5, li = lane & 31;
-
-  const TileCoord tc = mm_tile_coord(g);
-  const int64_t m0 = tc.m0, n0 = tc.n0;
-  const float *A = tc.A;
-  const float *B = tc.B;
-
-  floatx16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        acc[i][j][r] = 0.f;
-
-  TileLoad<LA> la;
-  TileLoad<LB> lb;
-  const int64_t ktiles = (g.K + MM_BK - 1) / MM_BK;
-  la.load(A, m0, 0, g.M, g.K, g.sAm, g.sAk, t);
-  lb.load(B, n0, 0, g.N, g.K, g.sBn, g.sBk, t);
-  la.store(lds[0][0], t);
-  lb.store(lds[0][1], t);
-  __syncthreads();
-
-  for (int64_t kt = 0; kt < ktiles; ++kt) {
-    const int cur = int(kt & 1);
-    if (kt + 1 < ktiles) {
-      la.load(A, m0, (kt + 1) * MM_BK, g.M, g.K, g.sAm, g.sAk, t);
-      lb.load(B, n0, (kt + 1) * MM_BK, g.N, g.K, g.sBn, g.sBk, t);
-    }
-    const float *As = lds[cur][0];
-    const float *Bs = lds[cur][1];
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      const int k = h * 16 + kk;
-      float a[2], b[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        a[i] = frag<LA>(As, wm * 64 + i * 32 + li, k);
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        b[j] = frag<LB>(Bs, wn * 64 + j * 32 + li, k);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j],
-                                                           acc[i][j], 0, 0, 0);
-    }
-    if (kt + 1 < ktiles) {
-      la.store(lds[cur ^ 1][0], t);
-      lb.store(lds[cur ^ 1][1], t);
-    }
-    __syncthreads();
+// One finished value of the product: to its slice's partial array, or to C
+// (accumulated, or with the bias).
+__device__ __forceinline__ void mm_put(const MMArgs &g, const TileCoord &tc,
+                                       int64_t row, int64_t col, float v) {
+  if (g.part) {
+    const int64_t p = int64_t(tc.slice) * g.nbatch + tc.batch;
+    g.part[(p * g.M + row) * g.N + col] = v;
+  } else {
+    float *dst = tc.C + row * g.sCm + col * g.sCn;
+    *dst = g.accumulate ? (*dst + v) : (g.bias ? v + g.bias[col * g.sBias] : v);
   }
-
-  mm_epilogue(g, tc, acc, wm, wn, h, li);
 }
 
 // ------------------------------------------ direct-to-LDS staging (gfx950)
 
-// gfx950 can move 16 bytes per lane from global memory straight into LDS
-// (global_load_lds_dwordx4): lane L of a wave lands at LDS base + 16 L, with
-// the base wave-uniform.  The kernel below stages both operands that way --
-// no VGPR round trip, no LDS store instructions -- when both are in a vector
-// layout and K is a multiple of the 32-deep k-tile.  Each wave instruction
-// fills 1 KB of a stage:
-//   layout K : the stage is [128 mn][32 k] without padding, 16-byte chunks
-//              swizzled within a row (dl_swz) so that fragment reads are
-//              bank-conflict free.  One instruction covers 8 rows.
-//   layout MN: the stage is [32 k][128 mn]; one instruction covers 2 k rows.
+// gfx950 moves 16 or 4 bytes per lane from global memory straight into LDS
+// (global_load_lds): lane L of a wave lands at LDS base + 16 L (or 4 L), with
+// the base wave-uniform.  No VGPR round trip, no LDS store instructions.
+// An operand's stage is a [mn][32 k] or [32 k][mn] tile, where mn is m for A
+// and n for B:
+//   ST_K16 : k is unit-stride, 16-byte loads; rows of 32 k, no padding,
+//            16-byte chunks swizzled within a row (dl_swz) so that fragment
+//            reads are bank-conflict free.  One instruction covers 8 rows.
+//   ST_MN16: mn is unit-stride, 16-byte loads; k rows of mn.
+//   ST_K4  : any strides, 4-byte loads with consecutive lanes along k (for
+//            odd row lengths, unaligned views); two rows of 32 k and 4 pad
+//            floats per instruction, which keeps the 16-byte fragment reads
+//            of 16 rows on distinct banks.
+//   ST_MN4 : any strides, 4-byte loads with consecutive lanes along mn.
 // Rows (columns) past M (N) re-read the last valid one: their results are
 // never stored.
-constexpr int DL_STAGE = 128 * 32; // floats per operand stage
+enum { ST_K16 = 0, ST_MN16 = 1, ST_K4 = 2, ST_MN4 = 3 };
 
 // Chunk swizzle of a [mn][k] stage row.  A fragment read is a 16-byte read
 // per lane of one chunk from 16 consecutive rows (lanes li of a half-wave);
@@ -323,54 +164,119 @@ constexpr int DL_STAGE = 128 * 32; // floats per operand stage
 // collide: rocprof counted one LDS bank conflict per read.)
 __device__ __forceinline__ int dl_swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
-template <int LAY> struct DirectTile {
-  const float *src[4]; // this work-item's source for instruction j, k-tile 0
-  int64_t kstep;       // elements between two k-tiles
+template <int ST, int B> struct StageTile {
+  static constexpr int FLOATS = ST == ST_K4 ? B / 2 * 68 : B * MM_BK;
+  static constexpr bool WIDE = ST == ST_K16 || ST == ST_MN16;
+  static constexpr int NI = WIDE ? B / 32 : B / 8; // instructions per wave
+  static constexpr int LDS_STEP = WIDE ? 256 : (ST == ST_K4 ? 68 : 64);
+  // Where element (mn, k) of the tile lies in the stage.
+  __device__ __forceinline__ static int pos(int mn, int k) {
+    if constexpr (ST == ST_K16)
+      return mn * 32 + (((k >> 2) ^ dl_swz(mn)) << 2) + (k & 3);
+    else if constexpr (ST == ST_K4)
+      return (mn >> 1) * 68 + (mn & 1) * 32 + k;
+    else
+      return k * B + mn;
+  }
+  const char *base;  // element (mn0, k0) of the operand
+  uint32_t off[NI];  // byte offset of this lane's source, instruction j
+  int64_t kstep;     // bytes between two k-tiles
   __device__ __forceinline__ void init(const float *p, int64_t mn0, int64_t MN,
                                        int64_t s_mn, int64_t s_k, int wave,
                                        int lane) {
+    base = reinterpret_cast<const char *>(p + mn0 * s_mn);
+    kstep = 4 * MM_BK * s_k;
+    // the last row (16-byte group of rows) that may be read
+    const int64_t last = MN - mn0 - (ST == ST_MN16 ? 4 : 1);
+    const int lastc = int(last < B - 1 ? last : B - 1);
+    const uint32_t bm = uint32_t(4 * s_mn), bk = uint32_t(4 * s_k);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if constexpr (LAY == LAY_K) {
-        const int r = (wave * 4 + j) * 8 + lane / 8;
-        const int c = (lane % 8) ^ dl_swz(r);
-        const int64_t row = mn0 + r < MN ? mn0 + r : MN - 1;
-        src[j] = p + row * s_mn + 4 * c;
+    for (int j = 0; j < NI; ++j) {
+      const int q = wave * NI + j;
+      int mn, k;
+      if constexpr (ST == ST_K16) {
+        mn = q * 8 + lane / 8;
+        k = 4 * ((lane % 8) ^ dl_swz(mn));
+      } else if constexpr (ST == ST_MN16) {
+        const int flat = q * 256 + lane * 4;
+        k = flat / B;
+        mn = flat % B;
+      } else if constexpr (ST == ST_K4) {
+        mn = q * 2 + lane / 32;
+        k = lane % 32;
       } else {
-        const int kr = (wave * 4 + j) * 2 + lane / 32;
-        const int64_t mn = mn0 + 4 * (lane % 32) <= MN - 4
-                               ? mn0 + 4 * (lane % 32)
-                               : MN - 4;
-        src[j] = p + kr * s_k + mn;
+        const int flat = q * 64 + lane;
+        k = flat / B;
+        mn = flat % B;
       }
+      mn = mn < lastc ? mn : lastc;
+      off[j] = uint32_t(mn) * bm + uint32_t(k) * bk;
     }
-    kstep = LAY == LAY_K ? 32 : 32 * s_k;
   }
   __device__ __forceinline__ void issue(float *stage, int64_t kt,
                                         int wave) const {
+    // Buffer loads: a scalar base and each lane's 32-bit offset.  (With
+    // global pointers the compiler kept a 64-bit address per load in
+    // registers and advanced them all each k-tile, and spilled in the
+    // 128x128 tiles.)  Every offset is in bounds by init's clamp; the range
+    // check of the resource is left wide open.
+    const char *src = base + kt * kstep;
+    const uint64_t ub = reinterpret_cast<uint64_t>(src);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(ub));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(uint32_t(ub >> 32));
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<void *>((uint64_t(hi) << 32) | lo), 0, -1, BUF_WORD3);
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void *)(src[j] + kt * kstep),
-          (__attribute__((address_space(3))) void *)(stage +
-                                                     (wave * 4 + j) * 256),
-          16, 0, 0);
+    for (int j = 0; j < NI; ++j) {
+      auto *to = (__attribute__((address_space(3))) void *)(stage +
+                                                            (wave * NI + j) * LDS_STEP);
+      if constexpr (WIDE)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, to, 16, int(off[j]), 0, 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, to, 4, int(off[j]), 0, 0, 0);
+    }
+  }
+  // The partial k-tile of K % 32 leading elements k0 .. K - 1, the rest
+  // zero: through registers.  p: the operand.
+  __device__ __forceinline__ static void stage_tail(float *stage, const float *p,
+                                                    int64_t mn0, int64_t MN,
+                                                    int64_t s_mn, int64_t s_k,
+                                                    int64_t k0, int64_t K, int t) {
+    constexpr int E = B * MM_BK / MM_THREADS;
+    float v[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int flat = t + MM_THREADS * e;
+      constexpr bool KF = ST == ST_K16 || ST == ST_K4;
+      const int mn = KF ? flat / MM_BK : flat % B;
+      const int k = KF ? flat % MM_BK : flat / B;
+      v[e] = 0.f;
+      if (mn0 + mn < MN && k0 + k < K)
+        v[e] = p[(mn0 + mn) * s_mn + (k0 + k) * s_k];
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int flat = t + MM_THREADS * e;
+      constexpr bool KF = ST == ST_K16 || ST == ST_K4;
+      const int mn = KF ? flat / MM_BK : flat % B;
+      const int k = KF ? flat % MM_BK : flat / B;
+      stage[pos(mn, k)] = v[e];
+    }
   }
 };
 
-// f[i][kk] = element (mn + 32 i, h * 16 + kk) of a direct-loaded stage.
-template <int LAY>
-__device__ __forceinline__ void dl_frags(const float *stage, int mn, int li,
-                                         int h, float (&f)[2][16]) {
+// f[i][kk] = element (mn + 32 i, h * 16 + kk) of a stage.
+template <int ST, int B, int NB>
+__device__ __forceinline__ void tile_frags(const float *stage, int mn, int li,
+                                           int h, float (&f)[NB][16]) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < NB; ++i) {
     const int row = mn + 32 * i + li;
-    if constexpr (LAY == LAY_K) {
+    if constexpr (ST == ST_K16 || ST == ST_K4) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int pc = (4 * h + q) ^ dl_swz(row);
-        const float4 w =
-            *reinterpret_cast<const float4 *>(stage + row * 32 + pc * 4);
+        const float4 w = *reinterpret_cast<const float4 *>(
+            stage + StageTile<ST, B>::pos(row, h * 16 + 4 * q));
         f[i][4 * q + 0] = w.x;
         f[i][4 * q + 1] = w.y;
         f[i][4 * q + 2] = w.z;
@@ -379,26 +285,9 @@ __device__ __forceinline__ void dl_frags(const float *stage, int mn, int li,
     } else {
 #pragma unroll
       for (int kk = 0; kk < 16; ++kk)
-        f[i][kk] = stage[(h * 16 + kk) * 128 + row];
+        f[i][kk] = stage[(h * 16 + kk) * B + row];
     }
   }
-}
-
-template <int LA, int LB>
-__device__ __forceinline__ void dl_compute(const float *sa, const float *sb,
-                                           int wm, int wn, int li, int h,
-                                           floatx16 (&acc)[2][2]) {
-  float fa[2][16], fb[2][16];
-  dl_frags<LA>(sa, wm * 64, li, h, fa);
-  dl_frags<LB>(sb, wn * 64, li, h, fb);
-#pragma unroll
-  for (int kk = 0; kk < 16; ++kk)
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][kk], fb[j][kk],
-                                                         acc[i][j], 0, 0, 0);
 }
 
 // Keeps a stage's direct loads where the source issues them, ahead of the
@@ -416,20 +305,125 @@ __device__ __forceinline__ void dl_wait_and_sync() {
   __syncthreads();
 }
 
-// Same tiling and MFMA schedule as mm_f32_mfma_kernel, operands staged by
+// A BM x BN tile of a slice of K: 4 waves in a WM x WN grid, each a
+// (BM / WM) x (BN / WN) block of 32x32 MFMA blocks.  Operands staged by
 // direct loads into two named stage pairs (the k loop is unrolled by two so
-// that every LDS access names its stage at compile time).
-template <int LA, int LB>
-__global__ __launch_bounds__(MM_THREADS, 2) void mm_f32_mfma_dl_kernel(
-    MMArgs g) {
-  __shared__ __align__(16) float sA0[DL_STAGE], sB0[DL_STAGE];
-  __shared__ __align__(16) float sA1[DL_STAGE], sB1[DL_STAGE];
+// that every LDS access names its stage at compile time).  A K that is not a
+// multiple of 32 starts with its partial k-tile, staged through registers.
+//
+// Bound: the fp32 MFMA pipe for large products (4000^3 at 134 TFLOP/s of the
+// 149 that a large library product reaches here), HBM for a few rows against
+// a large matrix (8x4096x4096: 67 MB in 18.8 us with its sum pass, 3.6 TB/s),
+// and in between the number of workgroups: hence small tiles, which also
+// waste less on ragged edges, and the split of K.  The 4-byte stages cost
+// four times the load instructions of the 16-byte ones and run at 0.8 of
+// their rate; through registers, one strided element at a time, odd row
+// lengths had run at a fifth of it.
+template <int SA, int SB, int BM, int BN>
+__global__ __launch_bounds__(MM_THREADS, BM * BN >= 128 * 128 ? 2 : 3)
+void mm_f32_tile_kernel(MMArgs g) {
+  using TA = StageTile<SA, BM>;
+  using TB = StageTile<SB, BN>;
+  constexpr int WN = BM == BN ? 2 : (BM < BN ? 4 : 1), WM = 4 / WN;
+  constexpr int NM = BM / WM / 32, NN = BN / WN / 32;
+  __shared__ __align__(16) float sA0[TA::FLOATS], sB0[TB::FLOATS];
+  __shared__ __align__(16) float sA1[TA::FLOATS], sB1[TB::FLOATS];
+  const int t = threadIdx.x;
+  const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int h = lane >> 5, li = lane & 31;
+  const TileCoord tc = mm_tile_coord<BM, BN>(g);
+
+  floatx16 acc[NM][NN];
+#pragma unroll
+  for (int i = 0; i < NM; ++i)
+#pragma unroll
+    for (int j = 0; j < NN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        acc[i][j][r] = 0.f;
+
+  const int64_t k0 = int64_t(tc.slice) * g.kslice;
+  const int64_t klen = g.K - k0 < g.kslice ? g.K - k0 : g.kslice;
+  const int64_t full = klen / MM_BK;
+  const int64_t tail = klen % MM_BK ? 1 : 0; // only in the last slice
+  TA ta;
+  TB tb;
+  ta.init(tc.A + k0 * g.sAk, tc.m0, g.M, g.sAm, g.sAk, wave, lane);
+  tb.init(tc.B + k0 * g.sBk, tc.n0, g.N, g.sBn, g.sBk, wave, lane);
+
+  auto compute = [&](const float *sa, const float *sb) {
+    float fa[NM][16], fb[NN][16];
+    tile_frags<SA, BM, NM>(sa, wm * (BM / WM), li, h, fa);
+    tile_frags<SB, BN, NN>(sb, wn * (BN / WN), li, h, fb);
+#pragma unroll
+    for (int kk = 0; kk < 16; ++kk)
+#pragma unroll
+      for (int i = 0; i < NM; ++i)
+#pragma unroll
+        for (int j = 0; j < NN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+              fa[i][kk], fb[j][kk], acc[i][j], 0, 0, 0);
+  };
+
+  const int64_t steps = full + tail; // step 0 is the partial tile, if any
+  if (tail) {
+    const int64_t kt = k0 + full * MM_BK;
+    TA::stage_tail(sA0, tc.A, tc.m0, g.M, g.sAm, g.sAk, kt, g.K, t);
+    TB::stage_tail(sB0, tc.B, tc.n0, g.N, g.sBn, g.sBk, kt, g.K, t);
+  } else {
+    ta.issue(sA0, 0, wave);
+    tb.issue(sB0, 0, wave);
+  }
+  dl_wait_and_sync();
+  for (int64_t s = 0; s < steps; s += 2) {
+    if (s + 1 < steps) {
+      ta.issue(sA1, s + 1 - tail, wave);
+      tb.issue(sB1, s + 1 - tail, wave);
+    }
+    pin_issued_loads();
+    compute(sA0, sB0);
+    dl_wait_and_sync();
+    if (s + 1 >= steps)
+      break;
+    if (s + 2 < steps) {
+      ta.issue(sA0, s + 2 - tail, wave);
+      tb.issue(sB0, s + 2 - tail, wave);
+    }
+    pin_issued_loads();
+    compute(sA1, sB1);
+    dl_wait_and_sync();
+  }
+
+  // lane holds column li of each 32x32 block, rows 8*(r/4) + 4*h + (r%4)
+#pragma unroll
+  for (int i = 0; i < NM; ++i)
+#pragma unroll
+    for (int j = 0; j < NN; ++j) {
+      const int64_t col = tc.n0 + wn * (BN / WN) + j * 32 + li;
+      if (col >= g.N)
+        continue;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int64_t row =
+            tc.m0 + wm * (BM / WM) + i * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
+        if (row < g.M)
+          mm_put(g, tc, row, col, acc[i][j][r]);
+      }
+    }
+}
+
+// Any strides at all (64-bit offsets, through registers): operands whose
+// strides exceed the tile kernel's 32-bit offsets (a row stride past 2^22
+// elements), 128x128 tiles.
+__global__ __launch_bounds__(MM_THREADS, 2) void mm_f32_far_kernel(MMArgs g) {
+  constexpr int P = MM_BK + 4; // padded [mn][k] row
+  __shared__ __align__(16) float lds[2][128 * P];
   const int t = threadIdx.x;
   const int lane = t & 63, wave = t >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int h = lane >> 5, li = lane & 31;
-  const TileCoord tc = mm_tile_coord(g);
-
+  const TileCoord tc = mm_tile_coord<128, 128>(g);
   floatx16 acc[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -438,34 +432,57 @@ __global__ __launch_bounds__(MM_THREADS, 2) void mm_f32_mfma_dl_kernel(
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         acc[i][j][r] = 0.f;
-
-  DirectTile<LA> ta;
-  DirectTile<LB> tb;
-  ta.init(tc.A, tc.m0, g.M, g.sAm, g.sAk, wave, lane);
-  tb.init(tc.B, tc.n0, g.N, g.sBn, g.sBk, wave, lane);
-  const int64_t ktiles = g.K / 32;
-  ta.issue(sA0, 0, wave);
-  tb.issue(sB0, 0, wave);
-  dl_wait_and_sync();
-  for (int64_t kt = 0; kt < ktiles; kt += 2) {
-    if (kt + 1 < ktiles) {
-      ta.issue(sA1, kt + 1, wave);
-      tb.issue(sB1, kt + 1, wave);
+  for (int64_t k0 = 0; k0 < g.K; k0 += MM_BK) {
+    float va[16], vb[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int flat = t + MM_THREADS * e;
+      const int64_t mn = flat >> 5, k = k0 + (flat & 31);
+      va[e] = vb[e] = 0.f;
+      if (tc.m0 + mn < g.M && k < g.K)
+        va[e] = tc.A[(tc.m0 + mn) * g.sAm + k * g.sAk];
+      if (tc.n0 + mn < g.N && k < g.K)
+        vb[e] = tc.B[(tc.n0 + mn) * g.sBn + k * g.sBk];
     }
-    pin_issued_loads();
-    dl_compute<LA, LB>(sA0, sB0, wm, wn, li, h, acc);
-    dl_wait_and_sync();
-    if (kt + 1 >= ktiles)
-      break;
-    if (kt + 2 < ktiles) {
-      ta.issue(sA0, kt + 2, wave);
-      tb.issue(sB0, kt + 2, wave);
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int flat = t + MM_THREADS * e;
+      lds[0][(flat >> 5) * P + (flat & 31)] = va[e];
+      lds[1][(flat >> 5) * P + (flat & 31)] = vb[e];
     }
-    pin_issued_loads();
-    dl_compute<LA, LB>(sA1, sB1, wm, wn, li, h, acc);
-    dl_wait_and_sync();
+    __syncthreads();
+#pragma unroll
+    for (int kk = 0; kk < 16; ++kk) {
+      float a[2], b[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        a[i] = lds[0][(wm * 64 + i * 32 + li) * P + h * 16 + kk];
+        b[i] = lds[1][(wn * 64 + i * 32 + li) * P + h * 16 + kk];
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j],
+                                                           acc[i][j], 0, 0, 0);
+    }
   }
-  mm_epilogue(g, tc, acc, wm, wn, h, li);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int64_t col = tc.n0 + wn * 64 + j * 32 + li;
+      if (col >= g.N)
+        continue;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int64_t row =
+            tc.m0 + wm * 64 + i * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
+        if (row < g.M)
+          mm_put(g, tc, row, col, acc[i][j][r]);
+      }
+    }
 }
 
 // ---------------------------------------- wide tile (direct-to-LDS, gfx950)
@@ -594,7 +611,7 @@ __global__ __launch_bounds__(WD_THREADS, 1) void mm_f32_mfma_wide_kernel(
 
   WideDirectTile<LA> ta;
   WideDirectTile<LB> tb;
-  const int64_t k0 = int64_t(blockIdx.y) * g.kslice;
+  const int64_t k0 = int64_t(tc.slice) * g.kslice;
   ta.init(tc.A + k0 * g.sAk, tc.m0, g.sAm, g.sAk, wave, lane);
   tb.init(tc.B + k0 * g.sBk, tc.n0, g.sBn, g.sBk, wave, lane);
   // The slice is a multiple of 64: k-tiles come in pairs, one per stage,
@@ -629,70 +646,55 @@ __global__ __launch_bounds__(WD_THREADS, 1) void mm_f32_mfma_wide_kernel(
       for (int r = 0; r < 16; ++r) {
         const int64_t row =
             tc.m0 + wm * 128 + i * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
-        const float v = acc[i][j][r];
-        if (g.part) {
-          g.part[(int64_t(blockIdx.y) * g.M + row) * g.N + col] = v;
-        } else {
-          float *dst = tc.C + row * g.sCm + col * g.sCn;
-          *dst = g.accumulate ? (*dst + v) : (g.bias ? v + g.bias[col * g.sBias] : v);
-        }
+        mm_put(g, tc, row, col, acc[i][j][r]);
       }
     }
 }
 
-// C[m][n] (+)= part[0][m][n] + part[1][m][n] + ... in slice order (a fixed
-// order: the result does not depend on scheduling).  Four columns per
-// work-item; N is a multiple of 4.
-template <int S, bool VEC_C>
+// C[b][m][n] (+)= part[0][b][m][n] + part[1][b][m][n] + ... in slice order (a
+// fixed order: the result does not depend on scheduling).  V adjacent columns
+// per work-item; V == 4 needs N a multiple of 4 and 16-byte rows of C.
+template <int S, int V>
 __global__ __launch_bounds__(256) void mm_splitk_sum_kernel(
-    const float *__restrict__ part, int64_t M, int64_t N, float *C,
-    int64_t sCm, int64_t sCn, int accumulate, const float *__restrict__ bias,
-    int64_t sBias, FastDivU32 fdn4, uint32_t total) {
-  // one work-item per 4 columns of one row, in a one-shot grid; the S slice
+    MMArgs g, FastDivU32 fdn, FastDivU32 fdm, uint32_t total) {
+  // one work-item per V columns of one row, in a one-shot grid; the S slice
   // loads are independent (S is a template argument) and go out together
   const uint32_t q = blockIdx.x * 256u + threadIdx.x;
   if (q >= total)
     return;
-  const uint32_t n4 = uint32_t(N / 4);
-  const uint32_t m32 = fdn4.div(q);
-  const int64_t m = m32, n = int64_t(q - m32 * n4) * 4;
-  typedef float f4 __attribute__((ext_vector_type(4)));
-  f4 w[S];
+  const uint32_t rm = fdn.div(q); // batch * M + m
+  const int64_t n = int64_t(q - rm * fdn.d) * V;
+  uint32_t batch = fdm.div(rm);
+  const int64_t m = rm - batch * uint32_t(g.M);
+  const int64_t slice = int64_t(g.nbatch) * g.M * g.N;
+  const float *p = g.part + int64_t(rm) * g.N + n;
+  typedef float fv __attribute__((ext_vector_type(V)));
+  fv w[S];
 #pragma unroll
   for (int s = 0; s < S; ++s)
     w[s] = __builtin_nontemporal_load(
-        reinterpret_cast<const f4 *>(part + (int64_t(s) * M + m) * N + n));
-  float4 v = make_float4(w[0].x, w[0].y, w[0].z, w[0].w);
+        reinterpret_cast<const fv *>(p + int64_t(s) * slice));
+  fv v = w[0];
 #pragma unroll
-  for (int s = 1; s < S; ++s) {
-    v.x = v.x + w[s].x;
-    v.y = v.y + w[s].y;
-    v.z = v.z + w[s].z;
-    v.w = v.w + w[s].w;
+  for (int s = 1; s < S; ++s)
+    v = v + w[s];
+  if (g.bias) // the product's value, then the bias add (its own rounding)
+#pragma unroll
+    for (int e = 0; e < V; ++e)
+      v[e] = v[e] + g.bias[(n + e) * g.sBias];
+  float *C = g.C;
+  for (int d = g.nb - 1; d >= 0; --d) {
+    const uint32_t sz = uint32_t(g.bshape[d]);
+    const uint32_t r = batch / sz;
+    C += int64_t(batch - r * sz) * g.bsC[d];
+    batch = r;
   }
-  if (bias) { // the product's value, then the bias add (its own rounding)
-    v.x = v.x + bias[(n + 0) * sBias];
-    v.y = v.y + bias[(n + 1) * sBias];
-    v.z = v.z + bias[(n + 2) * sBias];
-    v.w = v.w + bias[(n + 3) * sBias];
-  }
-  if constexpr (VEC_C) {
-    float4 *dst = reinterpret_cast<float4 *>(C + m * sCm + n);
-    if (accumulate) {
-      const float4 old = *dst;
-      v.x = old.x + v.x;
-      v.y = old.y + v.y;
-      v.z = old.z + v.z;
-      v.w = old.w + v.w;
-    }
-    *dst = v;
+  if constexpr (V > 1) {
+    fv *dst = reinterpret_cast<fv *>(C + m * g.sCm + n);
+    *dst = g.accumulate ? *dst + v : v;
   } else {
-    const float o[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float *dst = C + m * sCm + (n + e) * sCn;
-      *dst = accumulate ? (*dst + o[e]) : o[e];
-    }
+    float *dst = C + m * g.sCm + n * g.sCn;
+    *dst = g.accumulate ? *dst + v[0] : v[0];
   }
 }
 
@@ -749,89 +751,224 @@ __global__ __launch_bounds__(256) void mm_simt_kernel(MMArgsT<T> g) {
 
 namespace {
 
-template <int LA, int LB> void launch_mfma(const MMArgs &a, int64_t blocks) {
-  if constexpr (LA != LAY_GEN && LB != LAY_GEN) {
-    if (a.K % 32 == 0) {
-      // 256x256 tiles when they (or, for one product, they times a split of
-      // K into 2, 4 or 8 slices of at least 1024) give every CU one
-      const int64_t nbatch = blocks / (a.tiles_m * a.tiles_n);
-      MMArgs w = a;
-      w.tiles_m = (a.M + WD_BM - 1) / WD_BM;
-      w.tiles_n = (a.N + WD_BN - 1) / WD_BN;
-      const int64_t wblocks = w.tiles_m * w.tiles_n * nbatch;
-      const int64_t cus = device_cu_count();
-      if (a.M % WD_BM == 0 && a.N % WD_BN == 0 && a.K % 64 == 0) {
-        int S = 1;
-        while (wblocks * S < cus && nbatch == 1 && S < NT_MM_SPLITK_MAX &&
-               a.K % (64 * 2 * S) == 0 && a.K / (2 * S) >= 1024)
-          S *= 2;
-        if (wblocks * S >= cus) {
-          w.kslice = a.K / S;
-          if (S == 1) {
-            mm_f32_mfma_wide_kernel<LA, LB>
-                <<<dim3(unsigned(wblocks)), WD_THREADS, 0, stream()>>>(w);
-            return;
-          }
-          DeviceScratch part(size_t(S) * size_t(a.M) * size_t(a.N) *
-                             sizeof(float));
-          w.part = part.get<float>();
-          mm_f32_mfma_wide_kernel<LA, LB>
-              <<<dim3(unsigned(wblocks), unsigned(S)), WD_THREADS, 0,
-                 stream()>>>(w);
-          NT_LAUNCH_CHECK();
-          const int64_t items = a.M * (a.N / 4);
-          if (items >= (int64_t(1) << 32))
-            fail(NT_ERR_RUNTIME, "matmul: split-K output too large");
-          const unsigned grid = unsigned((items + 255) / 256);
-          const bool vec_c =
-              a.sCn == 1 && a.sCm % 4 == 0 &&
-              reinterpret_cast<uintptr_t>(a.C) % 16 == 0;
-          const FastDivU32 fdn4{uint32_t(a.N / 4)};
-#define NT_SPLITK_SUM(SS)                                                      \
-  do {                                                                         \
-    if (vec_c)                                                                 \
-      mm_splitk_sum_kernel<SS, true><<<grid, 256, 0, stream()>>>(              \
-          w.part, a.M, a.N, a.C, a.sCm, a.sCn, a.accumulate, a.bias, a.sBias,  \
-          fdn4, uint32_t(items));                                              \
-    else                                                                       \
-      mm_splitk_sum_kernel<SS, false><<<grid, 256, 0, stream()>>>(             \
-          w.part, a.M, a.N, a.C, a.sCm, a.sCn, a.accumulate, a.bias, a.sBias,  \
-          fdn4, uint32_t(items));                                              \
-  } while (0)
-          if (S == 2)
-            NT_SPLITK_SUM(2);
-          else if (S == 4)
-            NT_SPLITK_SUM(4);
-          else if (S == 8)
-            NT_SPLITK_SUM(8);
-          else
-            fail(NT_ERR_RUNTIME, "matmul: no split-K sum for this slice count");
-#undef NT_SPLITK_SUM
-          return;
-        }
-      }
-      mm_f32_mfma_dl_kernel<LA, LB>
-          <<<dim3(unsigned(blocks)), MM_THREADS, 0, stream()>>>(a);
-      return;
-    }
-  }
-  mm_f32_mfma_kernel<LA, LB>
-      <<<dim3(unsigned(blocks)), MM_THREADS, 0, stream()>>>(a);
-}
-
-template <int LA> void launch_mfma_b(int lb, const MMArgs &a, int64_t blocks) {
-  switch (lb) {
-  case LAY_K:
-    return launch_mfma<LA, LAY_K>(a, blocks);
-  case LAY_MN:
-    return launch_mfma<LA, LAY_MN>(a, blocks);
-  default:
-    return launch_mfma<LA, LAY_GEN>(a, blocks);
-  }
-}
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 bool aligned16(const void *p) {
   return reinterpret_cast<uintptr_t>(p) % 16 == 0;
+}
+
+// Runs `launch(args)` over S slices of K (each kslice long) into scratch and
+// adds them up; over one slice straight into C.  A split that the device
+// memory has no room for is not made.
+template <class F> void run_split(const MMArgs &a, int S, int64_t kslice, F launch) {
+  MMArgs w = a;
+  w.kslice = a.K;
+  w.part = nullptr;
+  const int64_t outs = int64_t(a.nbatch) * a.M * a.N;
+  if (S == 1 || outs >= (int64_t(1) << 32)) {
+    launch(w, 1);
+    return;
+  }
+  void *part = nullptr;
+  try {
+    part = device_alloc(size_t(S) * size_t(outs) * sizeof(float));
+  } catch (const Error &e) {
+    if (e.code != NT_ERR_OOM)
+      throw;
+    launch(w, 1);
+    return;
+  }
+  struct Free {
+    void *p;
+    ~Free() { device_free(p); }
+  } owner{part};
+  w.kslice = kslice;
+  w.part = static_cast<float *>(part);
+  launch(w, S);
+  NT_LAUNCH_CHECK();
+  bool vec = a.N % 4 == 0 && a.sCn == 1 && a.sCm % 4 == 0 && aligned16(a.C);
+  for (int d = 0; d < a.nb; ++d)
+    vec = vec && a.bsC[d] % 4 == 0;
+  const FastDivU32 fdn{uint32_t(vec ? a.N / 4 : a.N)}, fdm{uint32_t(a.M)};
+  const int64_t items = vec ? outs / 4 : outs;
+  const dim3 grid{unsigned(ceil_div(items, 256)), 1u, 1u};
+  auto sum = [&]<int SS>() {
+    if (vec)
+      mm_splitk_sum_kernel<SS, 4>
+          <<<grid, 256, 0, stream()>>>(w, fdn, fdm, uint32_t(items));
+    else
+      mm_splitk_sum_kernel<SS, 1>
+          <<<grid, 256, 0, stream()>>>(w, fdn, fdm, uint32_t(items));
+  };
+  switch (S) {
+  case 2:
+    return sum.template operator()<2>();
+  case 3:
+    return sum.template operator()<3>();
+  case 4:
+    return sum.template operator()<4>();
+  case 6:
+    return sum.template operator()<6>();
+  case 8:
+    return sum.template operator()<8>();
+  case 12:
+    return sum.template operator()<12>();
+  case 16:
+    return sum.template operator()<16>();
+  default:
+    fail(NT_ERR_RUNTIME, "matmul: no split-K sum for this slice count");
+  }
+}
+
+// Tile shape and slices of K of mm_f32_tile_kernel for one product: the
+// lowest estimated time.  The estimate, in us, is the k-tiles of one slice
+// times the larger of the MFMA time of the workgroups that share a CU and
+// the latency of a k-tile's loads (which up to 4 resident workgroups, or 2 of
+// the 128x128 tile, hide for each other), plus an epilogue per workgroup and
+// the pass that adds the slices.  The constants were fitted to 1700 timings:
+// 80 products from 16x16x10 to 8192x4096x1000, single and batched, in every
+// tile shape and split; over those products the choice is 1.0% slower than
+// the best one on average and 13% at worst (a 9 us product).  Before, one
+// 128x128 tile per workgroup and no split: 64x784x256 59 us, now 10; 8x4096
+// x4096 259 -> 19; 1000x784x1000 59 -> 20; 1537x1023x777 (odd rows) 174 ->
+// 35; 4000^3 1035 -> 951 (the 32-bit offsets of the staging loads).
+struct TileChoice {
+  int bm, bn, S;
+  int64_t kslice;
+};
+
+TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int64_t nbatch) {
+  constexpr double TK128 = 2.3, TK = 1.8; // us per 128x128x32 of MFMAs on a CU
+  constexpr double LAT128 = 0.65, LAT = 0.49, EPI = 1.07;
+  constexpr double SUM = 2.2, SUM_BYTES = 8.8e6; // us, bytes per us
+  constexpr double SCRATCH = 64 << 20; // a split's partial results
+  constexpr int SPLITS[] = {1, 2, 3, 4, 6, 8, 12, 16}; // as in run_split
+  const int64_t cus = device_cu_count();
+  const double outs = double(M) * double(N) * double(nbatch);
+  const int64_t kt = ceil_div(K, MM_BK);
+  int64_t kts[8]; // k-tiles of a slice, 0: no such split
+  double sum[8];  // the pass that adds the slices
+  for (int i = 0; i < 8; ++i) {
+    const int S = SPLITS[i];
+    const int64_t n = ceil_div(kt, S);
+    const bool ok = S == 1 || (n * (S - 1) < kt && S * outs * sizeof(float) <= SCRATCH);
+    kts[i] = ok ? n : 0;
+    sum[i] = S == 1 ? 0 : SUM + (S + 1) * outs * (sizeof(float) / SUM_BYTES);
+  }
+  static constexpr int SHAPES[][2] = {{128, 128}, {64, 64}, {32, 128}, {128, 32}};
+  TileChoice best{128, 128, 1, K};
+  double best_t = std::numeric_limits<double>::infinity();
+  for (const auto &sh : SHAPES) {
+    const int bm = sh[0], bn = sh[1];
+    const bool big = bm == 128 && bn == 128;
+    const double area = bm * bn / (128. * 128.);
+    const int64_t tiles = ceil_div(M, bm) * ceil_div(N, bn) * nbatch;
+    for (int i = 0; i < 8; ++i) {
+      if (kts[i] == 0)
+        continue;
+      const int64_t per_cu = ceil_div(tiles * SPLITS[i], cus);
+      const double mfma = double(per_cu) * (big ? TK128 : TK) * area;
+      const double lat = double(big ? (per_cu + 1) / 2 : (per_cu + 3) / 4) *
+                         (big ? LAT128 : LAT);
+      const double t =
+          double(kts[i]) * std::max(mfma, lat) + double(per_cu) * EPI * area + sum[i];
+      if (t < best_t) {
+        best_t = t;
+        best = {bm, bn, SPLITS[i], i == 0 ? K : kts[i] * MM_BK};
+      }
+    }
+  }
+  return best;
+}
+
+template <int SA, int SB, int BM, int BN>
+void launch_tile(const MMArgs &a, const TileChoice &c) {
+  run_split(a, c.S, c.kslice, [](MMArgs w, int S) {
+    w.tiles_m = ceil_div(w.M, BM);
+    w.tiles_n = ceil_div(w.N, BN);
+    const int64_t blocks = w.tiles_m * w.tiles_n * w.nbatch * S;
+    if (blocks >= (int64_t(1) << 31))
+      fail(NT_ERR_RUNTIME, "matmul: problem too large");
+    mm_f32_tile_kernel<SA, SB, BM, BN>
+        <<<dim3(unsigned(blocks)), MM_THREADS, 0, stream()>>>(w);
+  });
+}
+
+template <int SA, int SB> void launch_stages(const MMArgs &a) {
+  const TileChoice c = choose_tile(a.M, a.N, a.K, a.nbatch);
+  if (c.bm == 64)
+    launch_tile<SA, SB, 64, 64>(a, c);
+  else if (c.bm == 32)
+    launch_tile<SA, SB, 32, 128>(a, c);
+  else if (c.bn == 32)
+    launch_tile<SA, SB, 128, 32>(a, c);
+  else
+    launch_tile<SA, SB, 128, 128>(a, c);
+}
+
+template <int LA, int LB> bool launch_wide(const MMArgs &a) {
+  // 256x256 tiles when they (or, for one product, they times a split of
+  // K into 2, 4 or 8 slices of at least 1024) give every CU one
+  if (a.M % WD_BM != 0 || a.N % WD_BN != 0 || a.K % 64 != 0)
+    return false;
+  const int64_t tiles = a.M / WD_BM * (a.N / WD_BN) * a.nbatch;
+  const int64_t cus = device_cu_count();
+  int S = 1;
+  while (tiles * S < cus && a.nbatch == 1 && S < 8 && a.K % (64 * 2 * S) == 0 &&
+         a.K / (2 * S) >= 1024)
+    S *= 2;
+  if (tiles * S < cus)
+    return false;
+  run_split(a, S, a.K / S, [](MMArgs w, int slices) {
+    w.tiles_m = w.M / WD_BM;
+    w.tiles_n = w.N / WD_BN;
+    mm_f32_mfma_wide_kernel<LA, LB>
+        <<<dim3(unsigned(w.tiles_m * w.tiles_n * w.nbatch * slices)), WD_THREADS,
+           0, stream()>>>(w);
+  });
+  return true;
+}
+
+// fp32 product; al: both operands' bases and batch strides are 16-byte
+// aligned.
+void launch_f32(const MMArgs &a, bool al) {
+  // 16-byte loads need the unit-stride extent and the other stride to be
+  // multiples of 4 elements.
+  const bool ak = al && a.sAk == 1 && a.sAm % 4 == 0 && a.K % 4 == 0;
+  const bool am = al && a.sAm == 1 && a.sAk % 4 == 0 && a.M % 4 == 0;
+  const bool bn = al && a.sBn == 1 && a.sBk % 4 == 0 && a.N % 4 == 0;
+  const bool bk = al && a.sBk == 1 && a.sBn % 4 == 0 && a.K % 4 == 0;
+  const bool wide = (ak || am) && (bn || bk);
+  const bool a_mn = wide ? !ak : a.sAm < a.sAk;
+  const bool b_mn = wide ? bn : a.sBn < a.sBk;
+  if (wide && (a_mn ? (b_mn ? launch_wide<LAY_MN, LAY_MN>(a)
+                            : launch_wide<LAY_MN, LAY_K>(a))
+                    : (b_mn ? launch_wide<LAY_K, LAY_MN>(a)
+                            : launch_wide<LAY_K, LAY_K>(a))))
+    return;
+  constexpr int64_t FAR = int64_t(1) << 22;
+  if (a.sAm > FAR || a.sAk > FAR || a.sBn > FAR || a.sBk > FAR) {
+    MMArgs w = a;
+    w.kslice = a.K;
+    w.tiles_m = ceil_div(a.M, 128);
+    w.tiles_n = ceil_div(a.N, 128);
+    const int64_t blocks = w.tiles_m * w.tiles_n * w.nbatch;
+    if (blocks >= (int64_t(1) << 31))
+      fail(NT_ERR_RUNTIME, "matmul: problem too large");
+    mm_f32_far_kernel<<<dim3(unsigned(blocks)), MM_THREADS, 0, stream()>>>(w);
+    return;
+  }
+  if (wide) {
+    if (a_mn)
+      b_mn ? launch_stages<ST_MN16, ST_MN16>(a) : launch_stages<ST_MN16, ST_K16>(a);
+    else
+      b_mn ? launch_stages<ST_K16, ST_MN16>(a) : launch_stages<ST_K16, ST_K16>(a);
+  } else {
+    if (a_mn)
+      b_mn ? launch_stages<ST_MN4, ST_MN4>(a) : launch_stages<ST_MN4, ST_K4>(a);
+    else
+      b_mn ? launch_stages<ST_K4, ST_MN4>(a) : launch_stages<ST_K4, ST_K4>(a);
+  }
 }
 
 } // namespace
@@ -943,50 +1080,24 @@ void matmul_run(const nt_view *a, const nt_view *b, const nt_view *c,
       g.sCm = sCm;
       g.sCn = sCn;
       g.nb = nb;
-      bool batch_al = true;
+      bool al = aligned16(g.A) && aligned16(g.B);
       for (int d = 0; d < nb; ++d) {
         g.bshape[d] = a->shape[d];
         g.bsA[d] = st(a, d);
         g.bsB[d] = st(b, d);
         g.bsC[d] = st(c, d);
         if (g.bsA[d] % 4 != 0 || g.bsB[d] % 4 != 0)
-          batch_al = false;
+          al = false;
       }
+      if (nbatch >= (int64_t(1) << 31))
+        fail(NT_ERR_RUNTIME, "matmul: problem too large");
+      g.nbatch = uint32_t(nbatch);
       g.accumulate = accumulate ? 1 : 0;
       g.kslice = K;
       g.part = nullptr;
       g.bias = bias ? typed_ptr<const float>(bias) : nullptr;
       g.sBias = bias ? bias->strides[0] : 0;
-      // Vector (16-byte) tile loads need the unit-stride extent and the other
-      // stride to be multiples of 4 and a 16-byte aligned base.
-      int la = LAY_GEN, lb = LAY_GEN;
-      if (batch_al && aligned16(g.A)) {
-        if (sAk == 1 && sAm % 4 == 0 && K % 4 == 0)
-          la = LAY_K;
-        else if (sAm == 1 && sAk % 4 == 0 && M % 4 == 0)
-          la = LAY_MN;
-      }
-      if (batch_al && aligned16(g.B)) {
-        if (sBn == 1 && sBk % 4 == 0 && N % 4 == 0)
-          lb = LAY_MN;
-        else if (sBk == 1 && sBn % 4 == 0 && K % 4 == 0)
-          lb = LAY_K;
-      }
-      g.tiles_m = (M + MM_BM - 1) / MM_BM;
-      g.tiles_n = (N + MM_BN - 1) / MM_BN;
-      const int64_t blocks = g.tiles_m * g.tiles_n * nbatch;
-      if (blocks >= (int64_t(1) << 31))
-        fail(NT_ERR_RUNTIME, "matmul: problem too large");
-      switch (la) {
-      case LAY_K:
-        launch_mfma_b<LAY_K>(lb, g, blocks);
-        break;
-      case LAY_MN:
-        launch_mfma_b<LAY_MN>(lb, g, blocks);
-        break;
-      default:
-        launch_mfma_b<LAY_GEN>(lb, g, blocks);
-      }
+      launch_f32(g, al);
       NT_LAUNCH_CHECK();
       return;
     }

@@ -314,3 +314,56 @@ def test_matmul_bias_strided_operands(gpu):
         fused = host(nt.Tensor._new_contiguous(K.matmul_bias(ta, tb, tbias, (M, N)), (M, N)))
         prod = nt.Tensor._new_contiguous(K.matmul(ta, tb, (M, N)), (M, N))
         assert_bitexact(fused, host(prod + tbias), f"strided bias {M}x{K_}x{N}")
+
+
+# ------------------------------------------- tile shapes, splits, any layout
+
+# K below, at and past one k-tile of 32 and one unrolled pair; M and N on both
+# sides of the 32 / 64 / 128 tiles; few rows or columns against a large
+# matrix, and a small output over a long K (both split K); odd extents take
+# the 4-byte loads, multiples of 4 the 16-byte ones.
+TILE_SHAPES = [(1, 31, 257), (8, 2048, 1024), (3, 2047, 515), (31, 33, 129), (65, 64, 63),
+               (64, 2080, 64), (100, 2001, 36), (130, 65, 32), (1000, 784, 1000), (515, 4096, 9),
+               (257, 1023, 385)]
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("layout", ["NN", "TN", "NT", "TT"])
+@pytest.mark.parametrize("M,K_,N", TILE_SHAPES)
+def test_tile_kernel_edges(gpu, M, K_, N, layout, accumulate):
+    """Every output against the fp64 product.  fp32 sums of K products in any
+    order: |diff| <= K 2^-24 (|A|.|B|), times 2 for the slices' partial sums,
+    plus the accumulate's own rounding."""
+    r = rng(seed_of("tile", M, K_, N, layout, accumulate))
+    a = r.standard_normal((M, K_)).astype(np.float32)
+    b = (r.standard_normal((K_, N)) / np.sqrt(K_)).astype(np.float32)
+    old = r.standard_normal((M, N)).astype(np.float32)
+    tgt = dev(old)
+    K.matmul_into(dev_T(a) if layout[0] == "T" else dev(a),
+                  dev_T(b) if layout[1] == "T" else dev(b), tgt, accumulate=accumulate)
+    add = old if accumulate else 0.0
+    want = a.astype(np.float64) @ b + add
+    scale = np.abs(a).astype(np.float64) @ np.abs(b) + np.abs(add)
+    err = np.abs(host(tgt) - want) / scale
+    assert err.max() <= min(1e-4, 2 * (K_ + 2) * 2.0**-24), err.max()
+
+
+def test_tile_kernel_strided_outputs_and_batches(gpu):
+    """Split and unsplit products into transposed and sliced outputs, batched
+    with odd extents, and with row strides past the 32-bit load offsets."""
+    r = rng(seed_of("tile-views"))
+    for M, K_, N in ((40, 2000, 24), (40, 60, 24)):  # split, unsplit
+        a = r.standard_normal((M, K_)).astype(np.float32)
+        b = (r.standard_normal((K_, N)) / np.sqrt(K_)).astype(np.float32)
+        want = a.astype(np.float64) @ b
+        for tgt in (dev(np.zeros((N, M), np.float32)).T, dev(np.zeros((M, 2 * N), np.float32))[:, ::2]):
+            K.matmul_into(dev(a), dev(b), tgt, accumulate=False)
+            assert np.abs(host(tgt) - want).max() < 1e-4
+    a = r.standard_normal((2, 3, 33, 901)).astype(np.float32)  # batched, split, 4-byte loads
+    b = (r.standard_normal((2, 3, 901, 17)) / 30).astype(np.float32)
+    assert np.abs(_mm(dev(a), dev(b)) - a.astype(np.float64) @ b).max() < 1e-4
+    big = nt.zeros(6, 2**22 + 8, device="cuda")  # row stride past 2^22 elements
+    a = r.standard_normal((6, 40)).astype(np.float32)
+    big[:, 3:43] = dev(a)
+    b = (r.standard_normal((40, 9)) / 6).astype(np.float32)
+    assert np.abs(_mm(big[:, 3:43], dev(b)) - a.astype(np.float64) @ b).max() < 1e-4
