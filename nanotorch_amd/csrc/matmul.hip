@@ -33,7 +33,7 @@
 // bound).  Accumulate mode adds C_old after the full dot product: one
 // rounding, like the reference's `x._grad += grad`.
 //
-// Other dtypes (fp64, int32, int64) use a tiled SIMT kernel that accumulates
+// Other dtypes (fp64, int32, int64) use tiled SIMT kernels that accumulate
 // in k order exactly like the reference's CPU loop (matmul.cu:33-45).
 #include <algorithm>
 #include <limits>
@@ -712,41 +712,146 @@ template <class T> struct MMArgsT {
   int accumulate;
 };
 
-template <class T>
+// A (16 TM) x (16 TM) tile by 256 work-items of TM x TM outputs each, every
+// output summed in k order with the product and the sum rounded apart, as
+// the reference's loop does (no split of K, no FMA, no MFMA: their results
+// differ in the last bits).  Operands go through registers into [k][mn] LDS
+// stages, the next k-tile's loads in flight under this one's arithmetic.
+// Bound by the float64 instructions of the one wave that a tile gives each
+// SIMD (5.8 cycles each from a single wave, 4 from several; a multiply and an
+// add apart reach at most 39 TFLOP/s) and by LDS, where 2 TM values are read
+// for TM^2 products; so a work-item holds as many outputs as leave every CU
+// a tile (simt_tile).  float64 1000x784x1000: 225 us with one output per
+// work-item, 105 with 4 x 4 (15 TFLOP/s; 113 with a k-tile of 16 and no XCD
+// order, 125 with LDS reads at their use).
+template <class T, int TM>
 __global__ __launch_bounds__(256) void mm_simt_kernel(MMArgsT<T> g) {
-  constexpr int TS = 16;
-  __shared__ T As[TS][TS + 1];
-  __shared__ T Bs[TS][TS + 1];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int64_t row = int64_t(blockIdx.y) * TS + ty;
-  const int64_t col = int64_t(blockIdx.x) * TS + tx;
+  constexpr int TS = 16 * TM, BK = 32;
+  constexpr int P = TS + 2; // LDS row of a k: 16-byte aligned pairs
+  constexpr int E = TS * BK / 256; // values per work-item, operand and k-tile
+  __shared__ __align__(16) T As[2][BK][P], Bs[2][BK][P];
+  const int t = threadIdx.x;
+  const int tx = t & 15, ty = t >> 4;
+  // Each XCD (workgroups go to the 8 of them round-robin) takes one run of
+  // tiles, in groups of 4 tile-rows walked column by column: its L2 then
+  // holds few rows of A and few columns of B.
+  const uint32_t gx = gridDim.x, gy = gridDim.y, n_tiles = gx * gy;
+  uint32_t tile = blockIdx.y * gx + blockIdx.x;
+  tile = tile % 8 * (n_tiles / 8) + min(tile % 8, n_tiles % 8) + tile / 8;
+  const uint32_t g0 = tile / (4 * gx) * 4, rows = min(4u, gy - g0);
+  const uint32_t in = tile - g0 * gx;
+  const int64_t m0 = int64_t(g0 + in % rows) * TS, n0 = int64_t(in / rows) * TS;
   const T *A = g.A;
   const T *B = g.B;
   T *C = g.C;
-  int64_t rem = blockIdx.z;
+  uint32_t rem = blockIdx.z;
   for (int d = g.nb - 1; d >= 0; --d) {
-    const int64_t q = rem / g.bshape[d];
-    const int64_t c = rem - q * g.bshape[d];
+    const uint32_t sz = uint32_t(g.bshape[d]);
+    const uint32_t q = rem / sz;
+    const int64_t c = rem - q * sz;
     rem = q;
     A += c * g.bsA[d];
     B += c * g.bsB[d];
     C += c * g.bsC[d];
   }
-  T acc = T(0);
-  for (int64_t k0 = 0; k0 < g.K; k0 += TS) {
-    const int64_t ka = k0 + tx, kb = k0 + ty;
-    As[ty][tx] = (row < g.M && ka < g.K) ? A[row * g.sAm + ka * g.sAk] : T(0);
-    Bs[ty][tx] = (kb < g.K && col < g.N) ? B[kb * g.sBk + col * g.sBn] : T(0);
-    __syncthreads();
-    const int kmax = (g.K - k0) < TS ? int(g.K - k0) : TS;
-    for (int k = 0; k < kmax; ++k)
-      acc = acc + As[ty][k] * Bs[k][tx];
+  // consecutive work-items along the axis with the smaller stride
+  const bool a_mn = g.sAm < g.sAk, b_mn = g.sBn < g.sBk;
+  T va[E], vb[E];
+  auto load = [&](int64_t k0) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int f = t + 256 * e;
+      const int64_t ma = m0 + (a_mn ? f % TS : f / BK), ka = k0 + (a_mn ? f / TS : f % BK);
+      const int64_t nb = n0 + (b_mn ? f % TS : f / BK), kb = k0 + (b_mn ? f / TS : f % BK);
+      va[e] = ma < g.M && ka < g.K ? A[ma * g.sAm + ka * g.sAk] : T(0);
+      vb[e] = nb < g.N && kb < g.K ? B[nb * g.sBn + kb * g.sBk] : T(0);
+    }
+  };
+  auto store = [&](int s) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int f = t + 256 * e;
+      As[s][a_mn ? f / TS : f % BK][a_mn ? f % TS : f / BK] = va[e];
+      Bs[s][b_mn ? f / TS : f % BK][b_mn ? f % TS : f / BK] = vb[e];
+    }
+  };
+  // Output i of an axis: pairs of neighbours, 32 apart (a wave's reads of 16
+  // bytes per work-item are then contiguous).
+  auto at = [](int i, int q) { return TM == 1 ? q : (i / 2) * 32 + q * 2 + (i & 1); };
+  T acc[TM][TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+      acc[i][j] = T(0);
+  load(0);
+  store(0);
+  __syncthreads();
+  int s = 0;
+  for (int64_t k0 = 0; k0 < g.K; k0 += BK, s ^= 1) {
+    if (k0 + BK < g.K)
+      load(k0 + BK);
+    if (k0 + BK <= g.K) {
+      // Groups of U k's, each group's LDS reads issued before the previous
+      // group's arithmetic: a tile alone on its CU has one wave per SIMD,
+      // and nothing else would hide their latency.
+      constexpr int U = 4 / TM;
+      T a[2][U][TM], b[2][U][TM];
+      auto read = [&](int p, int k) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int i = 0; i < TM; ++i) {
+            a[p][u][i] = As[s][k + u][at(i, ty)];
+            b[p][u][i] = Bs[s][k + u][at(i, tx)];
+          }
+      };
+      read(0, 0);
+#pragma unroll
+      for (int k = 0; k < BK; k += U) {
+        const int p = k / U & 1;
+        if (k + U < BK)
+          read(p ^ 1, k + U);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          T c[TM][TM];
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TM; ++j)
+              c[i][j] = a[p][u][i] * b[p][u][j];
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TM; ++j)
+              acc[i][j] = acc[i][j] + c[i][j];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else { // no term past K (a zero operand times another is not always 0)
+#pragma unroll 1
+      for (int k = 0; k < int(g.K - k0); ++k)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TM; ++j)
+            acc[i][j] = acc[i][j] + As[s][k][at(i, ty)] * Bs[s][k][at(j, tx)];
+    }
+    if (k0 + BK < g.K)
+      store(s ^ 1);
     __syncthreads();
   }
-  if (row < g.M && col < g.N) {
-    T *dst = C + row * g.sCm + col * g.sCn;
-    *dst = g.accumulate ? T(*dst + acc) : acc;
-  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      const int64_t row = m0 + at(i, ty), col = n0 + at(j, tx);
+      if (row < g.M && col < g.N) {
+        T *dst = C + row * g.sCm + col * g.sCn;
+        *dst = g.accumulate ? T(*dst + acc[i][j]) : acc[i][j];
+      }
+    }
 }
 
 namespace {
@@ -904,6 +1009,23 @@ template <int SA, int SB> void launch_stages(const MMArgs &a) {
     launch_tile<SA, SB, 128, 32>(a, c);
   else
     launch_tile<SA, SB, 128, 128>(a, c);
+}
+
+// Outputs per work-item and axis of mm_simt_kernel: a k step of a tile costs
+// about TM units of LDS time (2 TM reads per work-item) for TM^2 outputs, so
+// the larger tile wins unless it leaves CUs without one.
+int simt_tile(int64_t M, int64_t N, int64_t nbatch) {
+  int best = 1;
+  int64_t best_t = std::numeric_limits<int64_t>::max();
+  for (int tm : {4, 2, 1}) {
+    const int64_t tiles = ceil_div(M, 16 * tm) * ceil_div(N, 16 * tm) * nbatch;
+    const int64_t t = ceil_div(tiles, device_cu_count()) * tm;
+    if (t < best_t) {
+      best_t = t;
+      best = tm;
+    }
+  }
+  return best;
 }
 
 template <int LA, int LB> bool launch_wide(const MMArgs &a) {
@@ -1126,9 +1248,21 @@ void matmul_run(const nt_view *a, const nt_view *b, const nt_view *c,
       g.accumulate = accumulate ? 1 : 0;
       if (nbatch > 65535)
         fail(NT_ERR_RUNTIME, "matmul: too many batches for the SIMT path");
-      dim3 grid{unsigned((N + 15) / 16), unsigned((M + 15) / 16),
-                unsigned(nbatch)};
-      mm_simt_kernel<T><<<grid, 256, 0, stream()>>>(g);
+      auto run = [&]<int TM>() {
+        const dim3 grid{unsigned(ceil_div(N, 16 * TM)), unsigned(ceil_div(M, 16 * TM)),
+                        unsigned(nbatch)};
+        mm_simt_kernel<T, TM><<<grid, 256, 0, stream()>>>(g);
+      };
+      switch (simt_tile(M, N, nbatch)) {
+      case 4:
+        run.template operator()<4>();
+        break;
+      case 2:
+        run.template operator()<2>();
+        break;
+      default:
+        run.template operator()<1>();
+      }
       NT_LAUNCH_CHECK();
     });
   }

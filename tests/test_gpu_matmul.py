@@ -367,3 +367,26 @@ def test_tile_kernel_strided_outputs_and_batches(gpu):
     big[:, 3:43] = dev(a)
     b = (r.standard_normal((40, 9)) / 6).astype(np.float32)
     assert np.abs(_mm(big[:, 3:43], dev(b)) - a.astype(np.float64) @ b).max() < 1e-4
+
+
+@pytest.mark.parametrize("layout", ["NN", "TN", "NT", "TT"])
+@pytest.mark.parametrize("M,K_,N", [(1000, 33, 993), (500, 70, 505), (33, 16, 65), (5, 1, 3)])
+@pytest.mark.parametrize("dt", [np.float64, np.int64, np.int32])
+def test_other_dtypes_exact_in_every_tile(gpu, M, K_, N, layout, dt):
+    """The 4x4, 2x2 and 1x1 register tiles (1000, 500 and 33 rows; K below,
+    at and past a k-tile) sum in k order with separate roundings: bit for bit
+    the oracle's loop, written and accumulated, also batched."""
+    r = rng(seed_of("simt", M, K_, N, layout, np.dtype(dt).name))
+    a = (r.standard_normal((M, K_)) * 100).astype(dt)
+    b = (r.standard_normal((K_, N)) * 100).astype(dt)
+    old = (r.standard_normal((M, N)) * 100).astype(dt)
+    xa = dev_T(a) if layout[0] == "T" else dev(a)
+    xb = dev_T(b) if layout[1] == "T" else dev(b)
+    want = O.matmul(a, b, parallel=True)
+    assert_bitexact(_mm(xa, xb), want, "product")
+    tgt = dev(old)
+    K.matmul_into(xa, xb, tgt, accumulate=True)
+    assert_bitexact(host(tgt), old + want, "accumulated")
+    if M < 100:
+        got = _mm(xa.reshape(1, M, K_).expand(3, M, K_), xb.reshape(1, K_, N).expand(3, K_, N))
+        assert_bitexact(got, np.broadcast_to(want, (3, M, N)), "batched")
