@@ -237,6 +237,14 @@ int nt_sgd_step(const nt_view *p, const nt_view *g, double lr);
 int nt_reduce(int32_t op, const nt_view *x, const int64_t *axes, int32_t naxes,
               const nt_view *out, const nt_view *idx, const nt_view *count);
 
+/* The mean over `axes` in one call: nt_reduce(NT_SUM) into out's dtype
+ * (float32 or float64), each sum then divided by the number of elements that
+ * it adds, which is MeanOp's sum and division
+ * (src/nanotorch/autograd/ops_reduction.py:107-127) with the same rounding
+ * after the sum. */
+int nt_mean(const nt_view *x, const int64_t *axes, int32_t naxes,
+            const nt_view *out);
+
 /* Bytes of the static device scratch array of the allocation-free entry
  * points (one array per GPU, held until the process ends). */
 #define NT_NOALLOC_SCRATCH_BYTES (16u << 20)

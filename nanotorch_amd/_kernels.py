@@ -246,6 +246,18 @@ def reduce(op: int, x, axes, out_dtype: Dtype, want_aux: bool = False):
     return out
 
 
+def mean(x, axes, out_dtype: Dtype) -> Storage:
+    """Mean over `axes`: the sum in out_dtype divided by the element count,
+    in one call (nt_mean)."""
+    require_device(x)
+    k = _numel([s for i, s in enumerate(x._shape) if i not in axes])
+    out = Storage.allocate(k, out_dtype, Device.Cuda)
+    vx = view_of(x)
+    vo = flat_view(out, (k,))
+    _lib.call("nt_mean", ctypes.byref(vx), _lib.axes_array(axes), len(axes), ctypes.byref(vo))
+    return out
+
+
 def reduce_bwd(op: int, g, scale: float, idx, cnt, axes, shape, target):
     """Backward of a reduction into a tensor of `shape`.  g holds one value
     per kept index (any shape, made contiguous here); accumulates into

@@ -107,14 +107,12 @@ class MeanOp(Function):
         self._x_dtype = x.dtype
         self._dtype = dtype
         new_shape = _out_shape(x, self._axis, keepdim)
-        if x.is_empty:
-            s = Tensor._new_contiguous(
-                K.fill(math.prod(new_shape), 0, dtype, x.device), new_shape
-            )
-        else:
-            s = Tensor._new_contiguous(K.reduce(_lib.R_SUM, x, self._axis, dtype), new_shape)
         self._orig_shape = x.shape
-        self._denom = x.numel // s.numel if s.numel else 0
+        n_out = math.prod(new_shape)
+        self._denom = x.numel // n_out if n_out else 0
+        if not x.is_empty:
+            return Tensor._new_contiguous(K.mean(x, self._axis, dtype), new_shape)
+        s = Tensor._new_contiguous(K.fill(n_out, 0, dtype, x.device), new_shape)
         if s.device == Device.Cpu:
             K.require_device(s)
         denom = _scalar_like(float(self._denom), dtype, s.device).expand(*s.shape)

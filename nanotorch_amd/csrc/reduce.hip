@@ -143,6 +143,7 @@ template <class O, bool IS_MAX> struct SelAcc {
       j = o.j;
       c = o.c;
     } else if (o.v == v) {
+      v = o.j < j ? o.v : v; // of two zeros, the first one's sign
       j = o.j < j ? o.j : j;
       c += o.c;
     }
@@ -239,16 +240,25 @@ template <class O, bool IS_MAX> struct ColLocal<SelAcc<O, IS_MAX>> {
   }
 };
 
+// Adds one in-walk chain of sums to another (max/min walk a single chain).
+template <class LA> __device__ __forceinline__ void merge_local(LA &a, const LA &b) {
+  if constexpr (requires { a.merge(b); })
+    a.merge(b);
+}
+
 // Writes the final accumulator of slice k.
 // MODE 0: sum value; 1: extremum value (+ optional idx/count); 2: index.
+// A mean's sum is divided by `count` (0: a plain sum) as it is written, the
+// same rounding as a division kernel after the sum.
 template <int MODE> struct RedOut {
   void *val;
   int64_t *idx;
   int32_t *cnt;
+  double count = 0;
   template <class O, class Acc>
   __device__ __forceinline__ void write(int64_t k, const Acc &a) const {
     if constexpr (MODE == 0) {
-      static_cast<O *>(val)[k] = a.s;
+      static_cast<O *>(val)[k] = count != 0 ? O(a.s / O(count)) : a.s;
     } else if constexpr (MODE == 1) {
       static_cast<O *>(val)[k] = a.v;
       if (idx)
@@ -289,12 +299,12 @@ struct KeepDesc {
   int64_t strides[NT_MAX_DIMS];
   __device__ __forceinline__ int64_t offset_of(int64_t k) const {
     int64_t off = 0;
-    for (int d = ndim - 1; d >= 0; --d) {
+    for (int d = ndim - 1; d >= 1; --d) {
       const int64_t q = k / shape[d];
       off += (k - q * shape[d]) * strides[d];
       k = q;
     }
-    return off;
+    return ndim > 0 ? off + k * strides[0] : off;
   }
 };
 
@@ -417,25 +427,32 @@ __global__ __launch_bounds__(RED_THREADS) void reduce_row_kernel(
   }
 }
 
-// x is [D, K] with K contiguous (stride 1) and row stride sd.  Block
-// (bx, s) covers columns [bx * CB, +CB), CB = 64 * VEC * WC, and rows
-// s, s + S, s + 2S, ...: WC waves stand side by side (lane l owns VEC
-// adjacent columns, so a block reads CB * sizeof(T) contiguous bytes of each
-// row) and the RED_WAVES / WC wave rows interleave the segment's rows, UR
-// rows in flight per lane.  Partials go to partial[s * K + k] (coalesced),
-// combined by reduce_col_combine_kernel.
-template <class T, class O, class Acc, int VEC, int WC, int UR, int MODE>
+// x is a batch (stride sb) of [D, K] matrices with K contiguous (stride 1)
+// and row stride sd.  Block (b nbx + bx, s) covers columns [bx * CB, +CB) of
+// matrix b, CB = CL * VEC * WC, and rows s, s + S, s + 2S, ...: CL lanes of a
+// wave times WC waves stand side by side (each lane owns VEC adjacent
+// columns, so a block reads CB * sizeof(T) contiguous bytes of each row), and
+// the WR = (64 / CL) (RED_WAVES / WC) wave rows interleave the segment's rows,
+// UR rows in flight per lane.  CL = 64 is for wide matrices; 16 and 4 keep the
+// lanes busy on narrow ones.  Partials go to partial[(s * batches + b) * K +
+// k] (coalesced), combined by reduce_col_combine_kernel.
+template <class T, class O, class Acc, int VEC, int WC, int CL, int UR, int MODE>
 __global__ __launch_bounds__(RED_THREADS) void reduce_col_kernel(
-    const T *__restrict__ x, int64_t K, int64_t D, int64_t sd, int S,
-    Acc *partial, RedOut<MODE> out) {
-  constexpr int WR = RED_WAVES / WC;
-  constexpr int CB = 64 * VEC * WC;
-  __shared__ Acc lds[WR > 1 ? RED_WAVES : 1][64 * VEC];
+    const T *__restrict__ x, int64_t K, int64_t D, int64_t sd, int64_t sb,
+    uint32_t nbx, int S, Acc *partial, RedOut<MODE> out) {
+  constexpr int LR = 64 / CL; // rows side by side in a wave
+  constexpr int WR = LR * (RED_WAVES / WC);
+  constexpr int CB = CL * VEC * WC;
+  __shared__ Acc lds[RED_WAVES > WC ? RED_WAVES : 1][CL * VEC];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int wc = w % WC, wr = w / WC;
+  const int wc = w % WC, wr = w / WC * LR + lane / CL;
+  const int cl = lane % CL;
   const int s = blockIdx.y;
-  const int64_t k0 =
-      int64_t(blockIdx.x) * CB + int64_t(wc) * 64 * VEC + int64_t(lane) * VEC;
+  const uint32_t batch = blockIdx.x / nbx;
+  const int64_t k0 = int64_t(blockIdx.x - batch * nbx) * CB +
+                     int64_t(wc) * CL * VEC + int64_t(cl) * VEC;
+  x += int64_t(batch) * sb;
+  const int64_t nk = int64_t(gridDim.x / nbx) * K; // kept indices in all
   // Segment s takes rows s, s + S, s + 2S, ... (relative row r is row
   // s + r S; D < 2^31, checked by the host), so all workgroups walk one
   // window of rows down the tensor together.  Contiguous row ranges per
@@ -447,10 +464,15 @@ __global__ __launch_bounds__(RED_THREADS) void reduce_col_kernel(
   const T *base = x + j0 * sd + k0;
   sd *= S;
   using LA = typename ColLocal<Acc>::type;
-  LA la[VEC];
+  // Sums: a chain per row of a group, merged pairwise below (each addend
+  // passes a quarter of the roundings of one chain per column).
+  constexpr int NA = IsSel<Acc>::value ? 1 : UR;
+  LA la[NA][VEC];
 #pragma unroll
-  for (int i = 0; i < VEC; ++i)
-    la[i].init();
+  for (int q = 0; q < NA; ++q)
+#pragma unroll
+    for (int i = 0; i < VEC; ++i)
+      la[q][i].init();
   using V = VecT<T, VEC>;
   if (k0 + VEC <= K) {
     int32_t jr = wr;
@@ -462,8 +484,8 @@ __global__ __launch_bounds__(RED_THREADS) void reduce_col_kernel(
     // between them would wait for the loads in flight).  The last prefetch
     // re-reads the last group (clamped index, in bounds) and is discarded.
     constexpr int32_t GR = UR * WR;
-    // wave-uniform loop control and addresses (scalar registers)
-    const int32_t wru = __builtin_amdgcn_readfirstlane(wr);
+    // (CL == 64: wave-uniform loop control and addresses, scalar registers)
+    const int32_t wru = CL == 64 ? __builtin_amdgcn_readfirstlane(wr) : wr;
     const int32_t nru = __builtin_amdgcn_readfirstlane(nr);
     const int32_t ng = nru - 1 - wru - (UR - 1) * WR >= 0
                            ? (nru - 1 - wru - (UR - 1) * WR) / GR + 1
@@ -483,7 +505,7 @@ __global__ __launch_bounds__(RED_THREADS) void reduce_col_kernel(
         for (int u = 0; u < UR; ++u)
 #pragma unroll
           for (int i = 0; i < VEC; ++i)
-            la[i].add(static_cast<O>(v[u].v[i]), jg + u * WR);
+            la[u % NA][i].add(static_cast<O>(v[u].v[i]), jg + u * WR);
       };
       auto at = [&](int32_t g) { return pa + int64_t(g < ng ? g : ng - 1) * gs; };
       load(va, pa);
@@ -511,85 +533,177 @@ __global__ __launch_bounds__(RED_THREADS) void reduce_col_kernel(
       for (int u = 0; u < UR; ++u)
 #pragma unroll
         for (int i = 0; i < VEC; ++i)
-          la[i].add(static_cast<O>(v[u].v[i]), jr + u * WR);
+          la[u % NA][i].add(static_cast<O>(v[u].v[i]), jr + u * WR);
     }
     for (; jr < nr; jr += WR) {
       const V v = vload<true, T, VEC>(base + int64_t(jr) * sd);
 #pragma unroll
       for (int i = 0; i < VEC; ++i)
-        la[i].add(static_cast<O>(v.v[i]), jr);
+        la[0][i].add(static_cast<O>(v.v[i]), jr);
     }
   } else if (k0 < K) {
     for (int32_t jr = wr; jr < nr; jr += WR)
       for (int i = 0; i < VEC; ++i)
         if (k0 + i < K)
-          la[i].add(static_cast<O>(base[int64_t(jr) * sd + i]), jr);
+          la[0][i].add(static_cast<O>(base[int64_t(jr) * sd + i]), jr);
   }
+#pragma unroll
+  for (int n = 1; n < NA; n *= 2)
+#pragma unroll
+    for (int q = 0; q + n < NA; q += 2 * n)
+#pragma unroll
+      for (int i = 0; i < VEC; ++i)
+        merge_local(la[q][i], la[q + n][i]);
   Acc a[VEC];
 #pragma unroll
   for (int i = 0; i < VEC; ++i)
-    a[i] = ColLocal<Acc>::widen(la[i], j0, jm);
-  if constexpr (WR > 1) {
-    // Wave rows of one column group merge in wave-row order.
+    a[i] = ColLocal<Acc>::widen(la[0][i], j0, jm);
+  // The rows side by side in a wave merge by shuffles, then the wave rows of
+  // one column group in wave-row order.
+#pragma unroll
+  for (int off = CL; off < 64; off <<= 1)
 #pragma unroll
     for (int i = 0; i < VEC; ++i)
-      lds[w][lane * VEC + i] = a[i];
+      a[i].shfl_merge(off);
+  if constexpr (RED_WAVES > WC) {
+    if (lane < CL)
+#pragma unroll
+      for (int i = 0; i < VEC; ++i)
+        lds[w][cl * VEC + i] = a[i];
     __syncthreads();
-    if (wr == 0) {
+    if (w / WC == 0)
 #pragma unroll
       for (int i = 0; i < VEC; ++i)
 #pragma unroll
-        for (int rr = 1; rr < WR; ++rr)
-          a[i].merge(lds[rr * WC + wc][lane * VEC + i]);
-    }
+        for (int rr = 1; rr < RED_WAVES / WC; ++rr)
+          a[i].merge(lds[rr * WC + wc][cl * VEC + i]);
   }
-  if (wr == 0) {
+  if (w / WC == 0 && lane < CL) {
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
-      const int64_t k = k0 + i;
+      const int64_t k = k0 + i, kk = int64_t(batch) * K + k;
       if (k < K) {
         if (S == 1)
-          out.template write<O>(k, a[i]);
+          out.template write<O>(kk, a[i]);
         else
-          partial[int64_t(s) * K + k] = a[i];
+          partial[int64_t(s) * nk + kk] = a[i];
       }
     }
   }
 }
 
-// Combines partial[s * K + k] over s for 64 columns per block: wave w
-// merges s = w, w + 4, ... (UR loads in flight), then the four waves merge
-// in order through LDS.
-template <class O, class Acc, int MODE>
+// Short contiguous slices (x + keep.offset_of(k)), one group of G lanes each,
+// 64 / G slices per wave.  Bound by HBM.  A workgroup per slice
+// (reduce_row_kernel) has no element for most of its work-items there and
+// spends its time on the LDS combine: along the last axis of [65536, 1024]
+// (268 MB) sum 62 -> 38.5 us, max with index and count 107 -> 39.9.
+template <class T, class O, class Acc, int VEC, int G, int MODE>
+__global__ __launch_bounds__(RED_THREADS) void reduce_short_rows_kernel(
+    const T *__restrict__ x, KeepDesc keep, int64_t K, int32_t D,
+    RedOut<MODE> out) {
+  const int g = threadIdx.x % G;
+  const int64_t k = int64_t(blockIdx.x) * (RED_THREADS / G) + threadIdx.x / G;
+  using V = VecT<T, VEC>;
+  constexpr int UR = 4;
+  using LA = typename ColLocal<Acc>::type;
+  // Sums: one chain per load and vector lane, merged pairwise below, so that
+  // no addend passes more roundings than with a work-item per vector.
+  constexpr int NA = IsSel<Acc>::value ? 1 : UR * VEC;
+  LA a[NA];
+#pragma unroll
+  for (int q = 0; q < NA; ++q)
+    a[q].init();
+  if (k < K) {
+    const T *row = x + keep.offset_of(k);
+    // Whole vectors, UR at a time; in the last group the loads past the end
+    // repeat the last vector (they stay unconditional, so that all of a
+    // group go out together) and count for nothing.
+    const int32_t nv = D / VEC;
+    auto group = [&]<bool LAST>(int32_t q) {
+      V v[UR];
+#pragma unroll
+      for (int u = 0; u < UR; ++u) {
+        const int32_t qu = q + u * G;
+        v[u] = vload<true, T, VEC>(row + (!LAST || qu < nv ? qu : nv - 1) * VEC);
+      }
+#pragma unroll
+      for (int u = 0; u < UR; ++u) {
+        const bool in = !LAST || q + u * G < nv;
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) {
+          const O e = static_cast<O>(v[u].v[i]);
+          const int32_t j = (q + u * G) * VEC + i;
+          if constexpr (IsSel<Acc>::value) {
+            if (in)
+              a[0].add(e, j);
+          } else {
+            a[u * VEC + i].add(in ? e : O(0), j);
+          }
+        }
+      }
+    };
+    int32_t q = g;
+    for (; q + (UR - 1) * G < nv; q += UR * G)
+      group.template operator()<false>(q);
+    if (q < nv)
+      group.template operator()<true>(q);
+    // the last D % VEC elements, one to a lane
+    const int32_t j = nv * VEC + g;
+    if (VEC > 1 && g < VEC && j < D)
+      a[0].add(static_cast<O>(row[j]), j);
+  }
+#pragma unroll
+  for (int n = 1; n < NA; n *= 2)
+#pragma unroll
+    for (int q = 0; q + n < NA; q += 2 * n)
+      merge_local(a[q], a[q + n]);
+  Acc r = ColLocal<Acc>::widen(a[0], 0);
+#pragma unroll
+  for (int off = 1; off < G; off <<= 1)
+    r.shfl_merge(off);
+  if (g == 0 && k < K)
+    out.template write<O>(k, r);
+}
+
+// Combines partial[s * K + k] over s for CC columns per block: the 256 / CC
+// rows of work-items merge s = r, r + 256 / CC, ... (UR loads in flight), then
+// the rows of a wave merge by shuffles and the four waves in order through
+// LDS.  Few columns per block when there are many partials of each.
+template <class O, class Acc, int MODE, int CC>
 __global__ __launch_bounds__(RED_THREADS) void reduce_col_combine_kernel(
     const Acc *__restrict__ partial, int64_t K, int S, RedOut<MODE> out) {
-  constexpr int UR = 4;
-  __shared__ Acc lds[RED_WAVES][64];
+  constexpr int UR = 4, RR = RED_THREADS / CC;
+  __shared__ Acc lds[RED_WAVES][CC];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t k = int64_t(blockIdx.x) * 64 + lane;
+  const int c = threadIdx.x % CC;
+  const int64_t k = int64_t(blockIdx.x) * CC + c;
   Acc a;
   a.init();
   if (k < K) {
-    int s = w;
-    for (; s + RED_WAVES * (UR - 1) < S; s += RED_WAVES * UR) {
+    int s = threadIdx.x / CC;
+    for (; s + RR * (UR - 1) < S; s += RR * UR) {
       Acc t[UR];
 #pragma unroll
       for (int u = 0; u < UR; ++u)
-        t[u] = partial[int64_t(s + RED_WAVES * u) * K + k];
+        t[u] = partial[int64_t(s + RR * u) * K + k];
 #pragma unroll
       for (int u = 0; u < UR; ++u)
         a.merge(t[u]);
     }
-    for (; s < S; s += RED_WAVES)
+    for (; s < S; s += RR)
       a.merge(partial[int64_t(s) * K + k]);
   }
-  lds[w][lane] = a;
+#pragma unroll
+  for (int off = CC; off < 64; off <<= 1)
+    a.shfl_merge(off);
+  if (lane < CC)
+    lds[w][c] = a;
   __syncthreads();
-  if (w == 0 && k < K) {
-    Acc r = lds[0][lane];
+  if (w == 0 && lane < CC && k < K) {
+    Acc r = lds[0][c];
 #pragma unroll
     for (int i = 1; i < RED_WAVES; ++i)
-      r.merge(lds[i][lane]);
+      r.merge(lds[i][c]);
     out.template write<O>(k, r);
   }
 }
@@ -779,16 +893,55 @@ void run_reduce(const nt_view *x, const RedPlan &p, RedOut<MODE> out,
 
   const bool drop_contig =
       p.drop.ndim == 0 || (p.drop.ndim == 1 && p.drop.strides[0] == 1);
-  const bool col_layout = p.drop.ndim == 1 && p.keep.ndim == 1 &&
-                          p.keep.strides[0] == 1 && p.drop.strides[0] != 1 &&
-                          p.D < (int64_t(1) << 31);
+  // One reduced axis over a contiguous kept one, with at most one more kept
+  // axis outside (a batch: the middle axis of a 3-D tensor).
+  const bool col_layout = p.drop.ndim == 1 && p.keep.ndim >= 1 && p.keep.ndim <= 2 &&
+                          p.keep.strides[p.keep.ndim - 1] == 1 &&
+                          p.drop.strides[0] != 1 && p.D < (int64_t(1) << 31);
+
+  // Vector loads along a contiguous slice need every slice start (and
+  // segment start) VEC-aligned.
+  bool row_aligned = reinterpret_cast<uintptr_t>(xp) % (sizeof(T) * VEC) == 0;
+  for (int d = 0; d < p.keep.ndim; ++d)
+    if (p.keep.strides[d] % VEC != 0)
+      row_aligned = false;
+
+  // Short contiguous slices: a few lanes each.  Longer ones, whose 16-byte
+  // loads fill a workgroup, and few ones, which would leave CUs without a
+  // wave, take a workgroup or more each below.  Sum / argmax along the last
+  // axis, us, workgroup per slice -> a few lanes per slice: [16384, 4000]
+  // 40.4 / 59.6 -> 40.2 / 42.9, [8192, 5000] 26.0 / 27.5 -> 26.8 / 27.8,
+  // [8192, 7001] (4-byte loads) 43.5 / 47.8 -> 40.1 / 42.1, [64, 4000]
+  // 4.4 / 8.5 -> 4.8 / 8.4, [100000, 10] 83.9 / 132 -> 4.4 / 8.9.
+  if (FAST && drop_contig && p.D < (row_aligned ? 4096 : 8192) &&
+      p.K >= (p.D <= 1024 ? 64 : 1000)) {
+    const KeepDesc kd = to_keep_desc(p.keep);
+    auto go = [&]<int V, int G>() {
+      const int64_t blocks = ceil_div(p.K, RED_THREADS / G);
+      if (blocks >= (int64_t(1) << 31))
+        fail(NT_ERR_RUNTIME, "reduction too large");
+      reduce_short_rows_kernel<T, O, Acc, V, G, MODE>
+          <<<dim3(unsigned(blocks)), RED_THREADS, 0, st>>>(xp, kd, p.K,
+                                                           int32_t(p.D), out);
+      NT_LAUNCH_CHECK();
+    };
+    // lanes per slice: about two vectors for each
+    auto lanes = [&]<int V>() {
+      if (p.D > 32 * V)
+        go.template operator()<V, 64>();
+      else if (p.D > 8 * V)
+        go.template operator()<V, 16>();
+      else
+        go.template operator()<V, 4>();
+    };
+    if (row_aligned)
+      lanes.template operator()<VEC>();
+    else
+      lanes.template operator()<1>();
+    return;
+  }
 
   if (FAST && drop_contig) {
-    // Vector loads need every slice start and segment start VEC-aligned.
-    bool aligned = reinterpret_cast<uintptr_t>(xp) % (sizeof(T) * VEC) == 0;
-    for (int d = 0; d < p.keep.ndim; ++d)
-      if (p.keep.strides[d] % VEC != 0)
-        aligned = false;
     // Long slices are split so that about NT_ROW_WG_PER_CU workgroups per
     // CU stream.
     const int64_t row_target = int64_t(device_cu_count()) * NT_ROW_WG_PER_CU;
@@ -809,10 +962,10 @@ void run_reduce(const nt_view *x, const RedPlan &p, RedOut<MODE> out,
     // a max/min segment spans the slice (round-robin chunks)
     const bool idx32 = (IsSel<Acc>::value ? p.D : seg) < (int64_t(1) << 31);
     const dim3 grid{unsigned(blocks), 1u, 1u};
-    if (aligned && idx32)
+    if (row_aligned && idx32)
       reduce_row_kernel<T, O, Acc, VEC, MODE, true>
           <<<grid, RED_THREADS, 0, st>>>(xp, kd, p.D, seg, int(S), partial, out);
-    else if (aligned)
+    else if (row_aligned)
       reduce_row_kernel<T, O, Acc, VEC, MODE, false>
           <<<grid, RED_THREADS, 0, st>>>(xp, kd, p.D, seg, int(S), partial, out);
     else if (idx32)
@@ -827,54 +980,81 @@ void run_reduce(const nt_view *x, const RedPlan &p, RedOut<MODE> out,
   }
 
   if (FAST && col_layout) {
-    const int64_t K = p.keep.shape[0], D = p.drop.shape[0];
-    const int64_t sd = p.drop.strides[0];
+    const int64_t K = p.keep.shape[p.keep.ndim - 1], D = p.drop.shape[0];
+    const int64_t B = p.keep.ndim == 2 ? p.keep.shape[0] : 1;
+    const int64_t sd = p.drop.strides[0], sb = B > 1 ? p.keep.strides[0] : 0;
     const bool aligned =
         reinterpret_cast<uintptr_t>(xp) % (sizeof(T) * VEC) == 0 &&
-        sd % VEC == 0;
+        sd % VEC == 0 && sb % VEC == 0;
     const int vec = aligned ? VEC : 1;
-    // Wide tensors: WC waves side by side (64 * vec * WC columns per
-    // workgroup); narrow ones: 1 column group, 4 wave rows.
+    // Wide matrices: WC waves side by side (64 * vec * WC columns per
+    // workgroup); narrower ones a wave, a quarter or a sixteenth of one, with
+    // the other lanes on other rows ([65536, 10], argmax: 14.9 -> 11.7 us).
+    // The middle axis of [128, 512, 1024] (268 MB): sum 300 -> 41 us, max
+    // with index and count 302 -> 43, against one workgroup per output that
+    // read one element per row.
     constexpr int UR = IsSel<Acc>::value ? NT_COL_UR_SEL : NT_COL_UR;
     constexpr int WC = NT_COL_WC;
     const int wc = K >= WC * 64 * vec ? WC : 1;
-    const int64_t bx = ceil_div(K, int64_t(64) * vec * wc);
+    const int cl = K > 32 * vec ? 64 : (K > 8 * vec ? 16 : 4);
+    const int64_t nbx = ceil_div(K, int64_t(cl) * vec * wc), bx = nbx * B;
     // About one (sum) or two (max/min, larger partials) workgroups per CU:
     // fewer, longer row walks with UR loads in flight measured faster than
-    // many short ones, and keep the partials small.
+    // many short ones, and keep the partials small.  4-byte loads keep a
+    // quarter of the bytes in flight: four times the workgroups ([8192, 999]
+    // 9.9 -> 10.0 us, [64, 197, 767] 65 -> 10.2).
     const int64_t col_target =
-        int64_t(device_cu_count()) *
+        int64_t(device_cu_count()) * (vec == 1 ? 4 : 1) *
         (sizeof(Acc) <= 8 ? NT_COL_WG_SUM : NT_COL_WG_SEL);
     int64_t S = std::max<int64_t>(1, ceil_div(col_target, bx));
-    S = std::min<int64_t>(S, std::max<int64_t>(1, D / (UR * (RED_WAVES / wc))));
+    S = std::min<int64_t>(
+        S, std::max<int64_t>(1, D / (UR * (RED_WAVES / wc) * (64 / cl))));
     S = std::min<int64_t>(S, 65535);
     const int64_t seg = ceil_div(D, S);
     S = ceil_div(D, seg);
-    PartialBuf partial_buf(S > 1 ? sizeof(Acc) * K * S : 0, fixed);
-    Acc *partial = partial_buf.get<Acc>();
-    if (bx >= (int64_t(1) << 31))
-      fail(NT_ERR_RUNTIME, "reduction too large");
-    const dim3 grid{unsigned(bx), unsigned(S), 1u};
-    if (aligned && wc == WC)
-      reduce_col_kernel<T, O, Acc, VEC, WC, UR, MODE>
-          <<<grid, RED_THREADS, 0, st>>>(xp, K, D, sd, int(S), partial, out);
-    else if (aligned)
-      reduce_col_kernel<T, O, Acc, VEC, 1, UR, MODE>
-          <<<grid, RED_THREADS, 0, st>>>(xp, K, D, sd, int(S), partial, out);
-    else if (wc == WC)
-      reduce_col_kernel<T, O, Acc, 1, WC, UR, MODE>
-          <<<grid, RED_THREADS, 0, st>>>(xp, K, D, sd, int(S), partial, out);
-    else
-      reduce_col_kernel<T, O, Acc, 1, 1, UR, MODE>
-          <<<grid, RED_THREADS, 0, st>>>(xp, K, D, sd, int(S), partial, out);
-    NT_LAUNCH_CHECK();
-    if (S > 1) {
-      reduce_col_combine_kernel<O, Acc, MODE>
-          <<<dim3(unsigned(ceil_div(K, 64))), RED_THREADS, 0, st>>>(
-              partial, K, int(S), out);
+    if (bx < (int64_t(1) << 31)) {
+      PartialBuf partial_buf(S > 1 ? sizeof(Acc) * K * B * S : 0, fixed);
+      Acc *partial = partial_buf.get<Acc>();
+      const dim3 grid{unsigned(bx), unsigned(S), 1u};
+      auto go = [&]<int V, int W, int CL>() {
+        reduce_col_kernel<T, O, Acc, V, W, CL, UR, MODE>
+            <<<grid, RED_THREADS, 0, st>>>(xp, K, D, sd, sb, uint32_t(nbx),
+                                           int(S), partial, out);
+      };
+      auto lanes = [&]<int V>() {
+        if (wc == WC)
+          go.template operator()<V, WC, 64>();
+        else if (cl == 64)
+          go.template operator()<V, 1, 64>();
+        else if (cl == 16)
+          go.template operator()<V, 1, 16>();
+        else
+          go.template operator()<V, 1, 4>();
+      };
+      if (aligned)
+        lanes.template operator()<VEC>();
+      else
+        lanes.template operator()<1>();
       NT_LAUNCH_CHECK();
+      if (S > 1) {
+        auto combine = [&]<int CC>() {
+          reduce_col_combine_kernel<O, Acc, MODE, CC>
+              <<<dim3(unsigned(ceil_div(K * B, CC))), RED_THREADS, 0, st>>>(
+                  partial, K * B, int(S), out);
+        };
+        // (about one group of UR partials for each work-item)
+        if (S >= 256 && K * B <= 4096)
+          combine.template operator()<4>();
+        else if (S >= 32)
+          combine.template operator()<16>();
+        else
+          combine.template operator()<64>();
+        NT_LAUNCH_CHECK();
+      }
+      return;
     }
-    return;
+    if (B == 1)
+      fail(NT_ERR_RUNTIME, "reduction too large");
   }
 
   // generic
@@ -963,50 +1143,63 @@ __global__ __launch_bounds__(256) void sel_bwd_kernel(
 
 // Max/min backward when gx is contiguous and the reduced axes are the
 // trailing (MODE 0: k = i / C, j = i % C), leading (MODE 1: k = i % C,
-// j = i / C) or all (MODE 2: k = 0, j = i) dims in increasing order.  Each
-// work-item writes 4 consecutive elements with one 16-byte store.
+// j = i / C), all (MODE 2: k = 0, j = i) or adjacent middle dims (MODE 3:
+// i = (b R + j) C + c, k = b C + c) in increasing order.  Each work-item
+// writes 4 consecutive elements with one 16-byte store; a tail of fewer than
+// 4 goes one by one.  Serves what sel_bwd_2d_kernel does not: row lengths
+// that are not a multiple of 4 ([8192, 1999] along the last axis 35.6 ->
+// 18.8 us, element by element before).
 template <class T, bool ACC, int MODE>
 __global__ __launch_bounds__(256) void sel_bwd_vec_kernel(
     const T *__restrict__ g, const int64_t *__restrict__ idx,
-    const int32_t *__restrict__ cnt, T *gx, FastDivU32 fdC, uint32_t C,
-    int64_t n4) {
-  const int64_t stride = int64_t(gridDim.x) * 256;
-  // q0: the block's first vector this round (uniform: the store base)
-  for (int64_t q0 = int64_t(blockIdx.x) * 256; q0 < n4; q0 += stride) {
-    const int64_t q = q0 + threadIdx.x;
-    if (q >= n4)
-      break;
-    VecT<T, 4> o;
-    VecT<T, 4> old;
-    if constexpr (ACC)
-      old = vload<true, T, 4>(gx + 4 * q);
-    const uint32_t i0 = uint32_t(4 * q);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const uint32_t i = i0 + e;
-      int64_t k, j;
-      if constexpr (MODE == 0) {
-        const uint32_t qq = fdC.div(i);
-        k = qq;
-        j = i - qq * C;
-      } else if constexpr (MODE == 1) {
-        const uint32_t qq = fdC.div(i);
-        k = i - qq * C;
-        j = qq;
-      } else {
-        k = 0;
-        j = i;
-      }
-      const bool sel = (j == idx[k]) && (cnt[k] == 1);
-      const T t = g[k] * (sel ? T(1) : T(0));
-      if constexpr (ACC)
-        o.v[e] = old.v[e] + t;
-      else
-        o.v[e] = t;
+    const int32_t *__restrict__ cnt, T *gx, FastDivU32 fdC, FastDivU32 fdR,
+    int64_t n) {
+  // q0: the block's first vector (uniform: the store base)
+  const int64_t q0 = int64_t(blockIdx.x) * 256;
+  const int64_t q = q0 + threadIdx.x;
+  if (4 * q >= n)
+    return;
+  auto term = [&](uint32_t i) {
+    int64_t k, j;
+    if constexpr (MODE == 0) {
+      const uint32_t qq = fdC.div(i);
+      k = qq;
+      j = i - qq * fdC.d;
+    } else if constexpr (MODE == 1) {
+      const uint32_t qq = fdC.div(i);
+      k = i - qq * fdC.d;
+      j = qq;
+    } else if constexpr (MODE == 3) {
+      const uint32_t r = fdC.div(i), b = fdR.div(r);
+      k = int64_t(b) * fdC.d + (i - r * fdC.d);
+      j = r - b * fdR.d;
+    } else {
+      k = 0;
+      j = i;
     }
-    vstore_out<true, 1, TK_SELVEC, T, 4>(gx + 4 * q0, 4 * int64_t(threadIdx.x),
-                                         true, o);
+    const bool sel = (j == idx[k]) && (cnt[k] == 1);
+    return T(g[k] * (sel ? T(1) : T(0)));
+  };
+  const uint32_t i0 = uint32_t(4 * q);
+  if (4 * q + 4 > n) {
+    for (uint32_t i = i0; i < n; ++i)
+      gx[i] = ACC ? gx[i] + term(i) : term(i);
+    return;
   }
+  VecT<T, 4> o;
+  VecT<T, 4> old;
+  if constexpr (ACC)
+    old = vload<true, T, 4>(gx + 4 * q);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const T t = term(i0 + e);
+    if constexpr (ACC)
+      o.v[e] = old.v[e] + t;
+    else
+      o.v[e] = t;
+  }
+  vstore_out<true, 1, TK_SELVEC, T, 4>(gx + 4 * q0, 4 * int64_t(threadIdx.x),
+                                       true, o);
 }
 
 // Max/min backward on a contiguous [Rr, Cc] gx, Cc % 4 == 0.  MODE 0: slice
@@ -1015,6 +1208,8 @@ __global__ __launch_bounds__(256) void sel_bwd_vec_kernel(
 // columns 4 * (64 bx + l) .. +3 and the waves walk rows by * rpb + w, +4, ...
 // The slice's (g, idx, count) is loaded once per row (MODE 0) or once per
 // work-item (MODE 1), so the kernel is a plain 16-byte streaming write.
+// blockIdx.z is a batch of such matrices (MODE 1: a middle axis reduced; max
+// backward over the middle axis of [128, 512, 1024]: 136 -> 46 us).
 template <class T, bool ACC, int MODE>
 __global__ __launch_bounds__(256) void sel_bwd_2d_kernel(
     const T *__restrict__ g, const int64_t *__restrict__ idx,
@@ -1025,6 +1220,12 @@ __global__ __launch_bounds__(256) void sel_bwd_2d_kernel(
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
   const int64_t c = (int64_t(blockIdx.x) * 64 + lane) * 4;
+  if constexpr (MODE == 1) {
+    g += blockIdx.z * Cc;
+    idx += blockIdx.z * Cc;
+    cnt += blockIdx.z * Cc;
+    gx += blockIdx.z * Rr * Cc;
+  }
   const int64_t r0 = int64_t(blockIdx.y) * rpb;
   const int64_t r1 = r0 + rpb < Rr ? r0 + rpb : Rr;
   const bool live = c < Cc;
@@ -1121,7 +1322,7 @@ namespace {
 // allocation-free variant, nullptr to take partials from the allocator.
 void reduce_impl(int32_t op, const nt_view *x, const int64_t *axes,
                  int32_t naxes, const nt_view *out, const nt_view *idx,
-                 const nt_view *count, void *fixed) {
+                 const nt_view *count, void *fixed, bool mean = false) {
   {
     check_view(x, "reduction");
     check_view(out, "reduction");
@@ -1140,6 +1341,11 @@ void reduce_impl(int32_t op, const nt_view *x, const int64_t *axes,
       RedOut<0> ro{nullptr, nullptr, nullptr};
       ro.val = static_cast<char *>(out->data) +
                out->offset * int64_t(dtype_size(out->dtype));
+      if (mean) {
+        if (out->dtype != NT_FLOAT32 && out->dtype != NT_FLOAT64)
+          fail(NT_ERR_VALUE, "mean: float output only");
+        ro.count = double(p.D);
+      }
       dispatch_all(x->dtype, [&]<class T>() {
         dispatch_arith(out->dtype, [&]<class O>() {
           run_reduce<T, O, SumAcc<O>, 0>(x, p, ro, fixed);
@@ -1199,6 +1405,13 @@ int nt_reduce(int32_t op, const nt_view *x, const int64_t *axes, int32_t naxes,
               const nt_view *out, const nt_view *idx, const nt_view *count) {
   return guard(
       [&] { reduce_impl(op, x, axes, naxes, out, idx, count, nullptr); });
+}
+
+int nt_mean(const nt_view *x, const int64_t *axes, int32_t naxes,
+            const nt_view *out) {
+  return guard([&] {
+    reduce_impl(NT_SUM, x, axes, naxes, out, nullptr, nullptr, nullptr, true);
+  });
 }
 
 int nt_reduce_noalloc(int32_t op, const nt_view *x, const int64_t *axes,
@@ -1271,39 +1484,46 @@ int nt_reduce_bwd(int32_t op, const nt_view *g, double scale, const nt_view *idx
         numel(idx) != K || numel(count) != K || !is_contiguous(idx) ||
         !is_contiguous(count))
       fail(NT_ERR_RUNTIME, "reduction_bwd: bad idx/count");
-    // Vector path: contiguous, aligned gx whose reduced axes are the
-    // trailing, leading or all dims, in increasing order.
+    // Vector paths: contiguous, aligned gx whose reduced axes are adjacent
+    // dims in increasing order.
     {
-      bool inc = true;
+      bool inc = naxes > 0;
       for (int i = 1; i < naxes; ++i)
         if (axes[i] != axes[i - 1] + 1)
           inc = false;
-      const bool trailing = inc && naxes > 0 && axes[naxes - 1] == gx->ndim - 1;
-      const bool leading = inc && naxes > 0 && axes[0] == 0;
       const size_t es = dtype_size(gx->dtype);
-      const bool ok = is_contiguous(gx) && n % 4 == 0 &&
-                      n < (int64_t(1) << 32) &&
-                      reinterpret_cast<uintptr_t>(
-                          static_cast<char *>(gx->data) + gx->offset * es) %
-                              (4 * es) == 0;
-      int mode = -1;
-      int64_t Cdim = 1;
-      if (ok && trailing && leading) {
-        mode = 2;
-      } else if (ok && trailing && D % 4 == 0) {
-        mode = 0;
-        Cdim = D;
-      } else if (ok && leading && K % 4 == 0) {
-        mode = 1;
-        Cdim = K;
-      }
-      if (mode >= 0) {
+      if (inc && is_contiguous(gx) && n < (int64_t(1) << 32) &&
+          reinterpret_cast<uintptr_t>(static_cast<char *>(gx->data) +
+                                      gx->offset * es) %
+                  (4 * es) == 0) {
+        const bool trailing = axes[naxes - 1] == gx->ndim - 1;
+        const bool leading = axes[0] == 0;
+        int64_t batch = 1;
+        for (int d = 0; d < axes[0]; ++d)
+          batch *= gx->shape[d];
+        const int64_t inner = K / batch; // kept elements after the reduced ones
+        int mode = 3;
+        int64_t Cdim = inner;
+        if (trailing && leading) {
+          mode = 2;
+        } else if (trailing) {
+          mode = 0;
+          Cdim = D;
+        } else if (leading) {
+          mode = 1;
+        }
+        // Rows of whole vectors: one slice per row, or one per column (of a
+        // batch; narrow rows would leave most of its lanes idle).
+        const bool rows2d =
+            Cdim % 4 == 0 &&
+            (mode == 0 || mode == 1 ||
+             (mode == 3 && Cdim >= 128 && batch <= 65535));
         const FastDivU32 fd{static_cast<uint32_t>(Cdim)};
-        const int64_t n4 = n / 4;
+        const FastDivU32 fdr{static_cast<uint32_t>(D)};
         // one work-item per 16-byte group (a one-shot grid, like the
         // elementwise engine's: a grid-stride loop over 16 workgroups per CU
         // wrote the full-reduction gradient at 4.3 TB/s, this at 6.6)
-        const int64_t blocks = std::max<int64_t>(1, ceil_div(n4, 256));
+        const int64_t blocks = ceil_div(ceil_div(n, 4), 256);
         dispatch_float(g->dtype, [&]<class T>() {
           const T *gp = typed_ptr<const T>(g);
           const int64_t *ip = typed_ptr<const int64_t>(idx);
@@ -1311,22 +1531,37 @@ int nt_reduce_bwd(int32_t op, const nt_view *g, double scale, const nt_view *idx
           T *xp = typed_ptr<T>(gx);
           const dim3 grid{unsigned(blocks), 1u, 1u};
           hipStream_t st = stream();
-          const uint32_t Cu = uint32_t(Cdim);
-          if (mode == 2) {
-            if (acc)
-              sel_bwd_vec_kernel<T, true, 2>
-                  <<<grid, 256, 0, st>>>(gp, ip, cp, xp, fd, Cu, n4);
-            else
-              sel_bwd_vec_kernel<T, false, 2>
-                  <<<grid, 256, 0, st>>>(gp, ip, cp, xp, fd, Cu, n4);
+          if (!rows2d) {
+            auto go = [&]<int M>() {
+              if (acc)
+                sel_bwd_vec_kernel<T, true, M>
+                    <<<grid, 256, 0, st>>>(gp, ip, cp, xp, fd, fdr, n);
+              else
+                sel_bwd_vec_kernel<T, false, M>
+                    <<<grid, 256, 0, st>>>(gp, ip, cp, xp, fd, fdr, n);
+            };
+            switch (mode) {
+            case 0:
+              go.template operator()<0>();
+              break;
+            case 1:
+              go.template operator()<1>();
+              break;
+            case 2:
+              go.template operator()<2>();
+              break;
+            default:
+              go.template operator()<3>();
+            }
           } else {
-            const int64_t Cc = Cdim, Rr = n / Cdim;
+            const int64_t nb = mode == 3 ? batch : 1;
+            const int64_t Cc = Cdim, Rr = n / Cdim / nb;
             const int64_t bx = ceil_div(Cc, 256);
             const int64_t target = int64_t(device_cu_count()) * NT_SEL2D_WG;
             const int64_t by = std::max<int64_t>(
-                1, std::min<int64_t>(ceil_div(target, bx), ceil_div(Rr, 16)));
+                1, std::min<int64_t>(ceil_div(target, bx * nb), ceil_div(Rr, 16)));
             const int64_t rpb = ceil_div(Rr, by);
-            const dim3 g2{unsigned(bx), unsigned(ceil_div(Rr, rpb)), 1u};
+            const dim3 g2{unsigned(bx), unsigned(ceil_div(Rr, rpb)), unsigned(nb)};
 #define NT_SEL2D(ACC, MODE)                                                    \
   sel_bwd_2d_kernel<T, ACC, MODE><<<g2, 256, 0, st>>>(gp, ip, cp, xp, Rr, Cc, \
                                                       rpb)

@@ -356,3 +356,82 @@ def test_float64_split_walks(gpu, shape, axes):
         assert_bitexact(host(nt.Tensor._new_contiguous(idx, kshape)), O.reduce(aop, a, axes), f"f64 arg {op}")
         want_cnt = (a == np.expand_dims(want, axes)).sum(axis=axes).astype(np.int32)
         assert_bitexact(host(nt.Tensor._new_contiguous(cnt, kshape)), want_cnt, f"f64 count {op}")
+
+
+# Middle axes (a batch of column walks) and narrow leading ones: column counts
+# on both sides of 4 lanes, 16 lanes, a wave and four waves of 16-byte or
+# 4-byte loads; rows below and past a pipelined group, one row, and enough to
+# split.  Short contiguous slices: below, at and past the vectors of 4, 16 and
+# 64 lanes and their unrolled loads, odd lengths (4-byte loads), and around the
+# lengths and counts past which a workgroup takes a slice.
+WALK_CASES = ([((3, d, c), (1,)) for d in (1, 5, 197) for c in (4, 15, 16, 33, 64, 129, 260, 1024, 1030)]
+              + [((2, 3000, c), (1,)) for c in (8, 10, 520)]
+              + [((5000, c), (0,)) for c in (3, 10, 16, 40, 64, 132)]
+              + [((70, d), (1,)) for d in (1, 4, 10, 16, 31, 32, 33, 128, 129, 130, 255, 256, 1000, 1001,
+                                           1023, 1024, 1028, 2047)]
+              + [((1001, d), (1,)) for d in (1025, 2052, 4095, 4096, 4097)]
+              + [((9, 11, 20), (2,)), ((64, 7, 6), (2,))])
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("shape,axes", WALK_CASES)
+def test_walks_forward_and_backward(gpu, shape, axes, dtype):
+    """max / min values, first indices, tie counts and the gradient's routing
+    bit for bit (small integers: ties, zeros of both signs); sums of them
+    exact; mean = that sum divided by the count, bit for bit."""
+    r = rng(seed_of("walks", shape, axes, np.dtype(dtype).name))
+    a = r.integers(-9, 10, shape).astype(dtype)
+    a[r.random(shape) < 0.1] = -0.0
+    x = dev(a)
+    nd = nt.float32 if dtype == np.float32 else nt.float64
+    ax = axes[0]
+    kshape = tuple(s for i, s in enumerate(shape) if i not in axes)
+    as_t = lambda st: host(nt.Tensor._new_contiguous(st, kshape))
+    total = a.sum(axis=ax)
+    assert (as_t(K.reduce(_lib.R_SUM, x, axes, nd)) == total).all()
+    assert_bitexact(as_t(K.mean(x, axes, nd)), (total + dtype(0)) / dtype(shape[ax]), "mean")
+    g = r.standard_normal(kshape).astype(dtype)
+    for op, oop, aop in ((_lib.R_MAX, O.R_MAX, O.R_ARGMAX), (_lib.R_MIN, O.R_MIN, O.R_ARGMIN)):
+        v, idx, cnt = K.reduce(op, x, axes, nd, want_aux=True)
+        first = O.reduce(aop, a, axes)
+        ext = O.reduce(oop, a, axes)
+        hit = a == np.expand_dims(ext, ax)
+        assert_bitexact(as_t(v), ext, "value")
+        assert_bitexact(as_t(idx), first, "index")
+        assert_bitexact(as_t(cnt), hit.sum(axis=ax).astype(np.int32), "count")
+        assert_bitexact(as_t(K.reduce(aop, x, axes, nt.int64)), first, "arg")
+        want = np.where(hit & (hit.sum(axis=ax, keepdims=True) == 1), np.expand_dims(g, ax), dtype(0))
+        st = K.reduce_bwd(op, dev(g), 1.0, idx, cnt, axes, shape, None)
+        got = host(nt.Tensor._new_contiguous(st, shape))
+        assert (got == want).all()
+        old = r.integers(-9, 10, shape).astype(dtype)
+        tgt = dev(old)
+        K.reduce_bwd(op, dev(g), 1.0, idx, cnt, axes, shape, tgt)
+        assert (host(tgt) == old + want).all()
+    old = r.standard_normal(shape).astype(dtype)
+    tgt = dev(old)
+    K.reduce_bwd(_lib.R_MEAN, dev(g), float(shape[ax]), None, None, axes, shape, tgt)
+    gd = np.broadcast_to(np.expand_dims(g / dtype(shape[ax]), ax), shape)
+    assert_bitexact(host(tgt), old + gd, "mean backward, accumulated")
+    st = K.reduce_bwd(_lib.R_MEAN, dev(g), float(shape[ax]), None, None, axes, shape, None)
+    assert_bitexact(host(nt.Tensor._new_contiguous(st, shape)), gd, "mean backward")
+
+
+@pytest.mark.parametrize("dt", ["f32", "f64", "i32>f32"])
+@pytest.mark.parametrize("C", [8, 12, 7])
+def test_broadcast_over_a_middle_axis(gpu, C, dt):
+    """[B, 1, C] and [B, T, 1] operands against [B, T, C] (16-byte groups
+    when C is a multiple of the vector, elements otherwise), into contiguous
+    and sliced outputs."""
+    r = rng(seed_of("bcast-mid", C, dt))
+    np_dt = np.float64 if dt == "f64" else np.float32
+    a = r.integers(-99, 100, (3, 5, C)).astype(np_dt)
+    m = r.integers(-99, 100, (3, 1, C)).astype(np.int32 if dt == "i32>f32" else np_dt)
+    s = r.integers(-99, 100, (3, 5, 1)).astype(np_dt)
+    assert_bitexact(host(dev(a) - dev(m)), (a - m).astype(np_dt), "row per batch")
+    assert_bitexact(host(dev(a) * dev(s) + dev(m)), (a * s + m).astype(np_dt), "column and row")
+    big = np.zeros((3, 7, 5, C), np_dt)
+    t = dev(big)
+    t[:, 2] = dev(a) * dev(m).to(nt.float64 if dt == "f64" else nt.float32)
+    big[:, 2] = a * m
+    assert_bitexact(host(t), big, "sliced output")
