@@ -123,7 +123,9 @@ def _totensor(x, *, anchor: Tensor) -> Tensor:
 
     Device scalars are cached by (type, value): building one costs a
     synchronous host-to-device copy, and the same constants (1, -1, lr)
-    recur every step.  The cached tensors are internal and never written.
+    recur every step.  The cached tensors are internal and never written, so
+    each also carries its value for ops that need it on the host (an
+    exponent), which would otherwise wait for the device to read it back.
     """
     if isinstance(x, Tensor):
         return x
@@ -133,7 +135,9 @@ def _totensor(x, *, anchor: Tensor) -> Tensor:
         if t is None or t.version != 0:
             if len(_SCALAR_CACHE) > 1024:
                 _SCALAR_CACHE.clear()
-            t = Tensor(x, device=anchor.device)
+            host = Tensor(x)
+            t = host.to(anchor.device)
+            t._host_value = host.item()  # as stored: a float rounded to float32
             _SCALAR_CACHE[key] = t
         return t
     return Tensor(x, device=anchor.device)

@@ -35,13 +35,16 @@ _CTYPES = {
 }
 
 
+_SIZES = {d: ctypes.sizeof(c) for d, c in _CTYPES.items()}
+
+
 def ctype_of(dtype: Dtype):
     return _CTYPES[Dtype(dtype)]
 
 
 def sizeof(dtype: Dtype) -> int:
     """Bytes per element (reference: core.py:35-44)."""
-    return ctypes.sizeof(_CTYPES[Dtype(dtype)])
+    return _SIZES[dtype]
 
 
 def dtype_from_type(data: InputType) -> Dtype:
@@ -71,7 +74,8 @@ def promote_dtypes(*dtypes: Dtype) -> Dtype:
     """Compute the highest precision Dtype."""
     if not dtypes:
         return Dtype.Float32
-    return Dtype(max(dtypes))
+    top = max(dtypes)
+    return top if type(top) is Dtype else Dtype(top)
 
 
 bool_ = Dtype.Bool

@@ -7,10 +7,27 @@ from types import EllipsisType
 TensorShape = tuple[int, ...]
 
 
+def row_major_strides(shape: TensorShape) -> TensorShape:
+    """Element strides of a contiguous tensor."""
+    n = len(shape)
+    if n == 2:
+        return (shape[1], 1)
+    if n == 1:
+        return (1,)
+    strides = []
+    acc = 1
+    for s in reversed(shape):
+        strides.append(acc)
+        acc *= s
+    return tuple(reversed(strides))
+
+
 def broadcast_shapes(*shapes: TensorShape) -> TensorShape:
     """Right-aligned broadcast of shapes; RuntimeError if incompatible."""
     if not shapes:
         return tuple()
+    if len(shapes) == 2 and shapes[0] == shapes[1]:
+        return tuple(shapes[0])
     final = list(shapes[0])
     for s in shapes[1:]:
         s = list(s)

@@ -14,6 +14,7 @@ import math
 
 from . import _lib
 from ._data_type import Dtype
+from ._indexing import row_major_strides
 from ._storage import Storage
 from .cuda import Device
 
@@ -21,7 +22,7 @@ from .cuda import Device
 def require_device(*tensors) -> None:
     """Device ops run on the GPU only; host tensors are staging buffers."""
     for t in tensors:
-        if t.device != Device.Cuda:
+        if t._storage._device != Device.Cuda:
             raise RuntimeError(
                 "nanotorch_amd computes on the GPU: move tensors to "
                 "device='cuda' (host tensors only hold and transfer data)."
@@ -40,14 +41,20 @@ def view_of(t) -> _lib.NtView:
 
 
 def flat_view(storage: Storage, shape, offset: int = 0) -> _lib.NtView:
-    strides = []
-    acc = 1
-    for d in reversed(shape):
-        strides.append(acc)
-        acc *= d
     return _lib.make_view(
-        storage.data_ptr(), offset, int(storage.dtype), tuple(shape), tuple(reversed(strides))
+        storage.data_ptr(), offset, int(storage.dtype), tuple(shape), row_major_strides(shape)
     )
+
+
+def _packed(t) -> bytes:
+    """view_of as bytes, for _lib.call_packed."""
+    s = t._storage
+    return _lib.pack_view(s._ptr, t._offset, s._dtype, t._shape, t._strides)
+
+
+def _packed_flat(storage: Storage, shape) -> bytes:
+    """flat_view as bytes, for _lib.call_packed."""
+    return _lib.pack_view(storage._ptr, 0, storage._dtype, shape, row_major_strides(shape))
 
 
 def _numel(shape) -> int:
@@ -72,9 +79,9 @@ def fill(n: int, value, dtype: Dtype, device: Device) -> Storage:
 def unary(op: int, x, scalar: float = 0.0) -> Storage:
     require_device(x)
     out = Storage.allocate(_numel(x._shape), x.dtype, Device.Cuda)
-    vx = view_of(x)
-    vo = flat_view(out, x._shape)
-    _lib.call("nt_unary", op, ctypes.byref(vx), float(scalar), ctypes.byref(vo))
+    vx = _packed(x)
+    vo = _packed_flat(out, x._shape)
+    _lib.call_packed("nt_unary", op, vx, float(scalar), vo)
     return out
 
 
@@ -84,9 +91,9 @@ def binary(op: int, x1, x2) -> Storage:
         raise RuntimeError("_dispatch_binary: Expected two views of the same shape.")
     out_dtype = Dtype.Bool if op in (_lib.EQ, _lib.GT, _lib.GE) else x1.dtype
     out = Storage.allocate(_numel(x1._shape), out_dtype, Device.Cuda)
-    v1, v2 = view_of(x1), view_of(x2)
-    vo = flat_view(out, x1._shape)
-    _lib.call("nt_binary", op, ctypes.byref(v1), ctypes.byref(v2), ctypes.byref(vo))
+    v1, v2 = _packed(x1), _packed(x2)
+    vo = _packed_flat(out, x1._shape)
+    _lib.call_packed("nt_binary", op, v1, v2, vo)
     return out
 
 
@@ -95,16 +102,16 @@ def sgd_step(p, g, lr32: float) -> None:
     reference's `p -= p.grad * lr`, nn/optimizers.py:45-51); float32
     device tensors of one shape, lr32 already a float32 value."""
     require_device(p, g)
-    vp, vg = view_of(p), view_of(g)
-    _lib.call("nt_sgd_step", ctypes.byref(vp), ctypes.byref(vg), lr32)
+    vp, vg = _packed(p), _packed(g)
+    _lib.call_packed("nt_sgd_step", vp, vg, lr32)
     p._storage.bump_version()
 
 
 def inplace(op: int, out, other) -> None:
     """out = out (op) other, in place (reference: inplace_ops.cu:39-79)."""
     require_device(out, other)
-    vo, v2 = view_of(out), view_of(other)
-    _lib.call("nt_inplace", op, ctypes.byref(vo), ctypes.byref(v2))
+    vo, v2 = _packed(out), _packed(other)
+    _lib.call_packed("nt_inplace", op, vo, v2)
     out._storage.bump_version()
 
 
@@ -114,8 +121,8 @@ def copy_view(src, out) -> None:
     if out.device == Device.Cpu:
         _host_copy(src, out)
         return
-    vs, vo = view_of(src), view_of(out)
-    _lib.call("nt_copy", ctypes.byref(vs), ctypes.byref(vo))
+    vs, vo = _packed(src), _packed(out)
+    _lib.call_packed("nt_copy", vs, vo)
 
 
 def clone_contiguous(x) -> Storage:
@@ -127,9 +134,9 @@ def clone_contiguous(x) -> Storage:
             out.host_array()[: len(vals)] = vals
         return out
     if _numel(x._shape):
-        vs = view_of(x)
-        vo = flat_view(out, x._shape)
-        _lib.call("nt_copy", ctypes.byref(vs), ctypes.byref(vo))
+        vs = _packed(x)
+        vo = _packed_flat(out, x._shape)
+        _lib.call_packed("nt_copy", vs, vo)
     return out
 
 
@@ -145,9 +152,9 @@ def cast(storage: Storage, dtype: Dtype) -> Storage:
         return Storage.from_iterable(src, dtype, Device.Cpu)
     out = Storage.allocate(n, dtype, Device.Cuda)
     if n:
-        vs = flat_view(storage, (n,))
-        vo = flat_view(out, (n,))
-        _lib.call("nt_copy", ctypes.byref(vs), ctypes.byref(vo))
+        vs = _packed_flat(storage, (n,))
+        vo = _packed_flat(out, (n,))
+        _lib.call_packed("nt_copy", vs, vo)
     return out
 
 
@@ -155,9 +162,9 @@ def equals(x1, x2) -> bool:
     _check_same_device(x1, x2)
     if x1.device == Device.Cpu:
         return host_values(x1) == host_values(x2)
-    v1, v2 = view_of(x1), view_of(x2)
+    v1, v2 = _packed(x1), _packed(x2)
     res = ctypes.c_int32(0)
-    _lib.call("nt_equals", ctypes.byref(v1), ctypes.byref(v2), ctypes.byref(res))
+    _lib.call_packed("nt_equals", v1, v2, ctypes.byref(res))
     return bool(res.value)
 
 
@@ -168,15 +175,15 @@ def unary_bwd(op: int, g, saved, scalar: float, gx_target) -> "Storage | None":
     """Fused unary backward.  gx_target is an existing gradient tensor to
     accumulate into (in place) or None; returns the new storage when None."""
     require_device(g)
-    vg = view_of(g)
-    vs = view_of(saved) if saved is not None else None
+    vg = _packed(g)
+    vs = _packed(saved) if saved is not None else None
     if gx_target is None:
         out = Storage.allocate(_numel(g._shape), g.dtype, Device.Cuda)
-        vo = flat_view(out, g._shape)
-        _lib.call("nt_unary_bwd", op, ctypes.byref(vg), _lib.ref(vs), float(scalar), ctypes.byref(vo), 0)
+        vo = _packed_flat(out, g._shape)
+        _lib.call_packed("nt_unary_bwd", op, vg, vs, float(scalar), vo, 0)
         return out
-    vo = view_of(gx_target)
-    _lib.call("nt_unary_bwd", op, ctypes.byref(vg), _lib.ref(vs), float(scalar), ctypes.byref(vo), 1)
+    vo = _packed(gx_target)
+    _lib.call_packed("nt_unary_bwd", op, vg, vs, float(scalar), vo, 1)
     gx_target._storage.bump_version()
     return None
 
@@ -184,9 +191,9 @@ def unary_bwd(op: int, g, saved, scalar: float, gx_target) -> "Storage | None":
 def binary_bwd(op: int, g, a, b, need_a: bool, target_a, need_b: bool, target_b):
     """Fused binary backward; returns (new_storage_a | None, new_storage_b | None)."""
     require_device(g)
-    vg = view_of(g)
-    va = view_of(a) if a is not None else None
-    vb = view_of(b) if b is not None else None
+    vg = _packed(g)
+    va = _packed(a) if a is not None else None
+    vb = _packed(b) if b is not None else None
     outs = []
     views = []
     for need, target in ((need_a, target_a), (need_b, target_b)):
@@ -196,20 +203,20 @@ def binary_bwd(op: int, g, a, b, need_a: bool, target_a, need_b: bool, target_b)
         elif target is None:
             st = Storage.allocate(_numel(g._shape), g.dtype, Device.Cuda)
             outs.append(st)
-            views.append((flat_view(st, g._shape), 0))
+            views.append((_packed_flat(st, g._shape), 0))
         else:
             outs.append(None)
-            views.append((view_of(target), 1))
+            views.append((_packed(target), 1))
     (vga, acc_a), (vgb, acc_b) = views
-    _lib.call(
+    _lib.call_packed(
         "nt_binary_bwd",
         op,
-        ctypes.byref(vg),
-        _lib.ref(va),
-        _lib.ref(vb),
-        _lib.ref(vga),
+        vg,
+        va,
+        vb,
+        vga,
         acc_a,
-        _lib.ref(vgb),
+        vgb,
         acc_b,
     )
     for need, target in ((need_a, target_a), (need_b, target_b)):
@@ -228,19 +235,17 @@ def reduce(op: int, x, axes, out_dtype: Dtype, want_aux: bool = False):
     keep = [s for i, s in enumerate(x._shape) if i not in axes]
     k = _numel(keep)
     out = Storage.allocate(k, out_dtype, Device.Cuda)
-    vx = view_of(x)
-    vo = flat_view(out, (k,))
+    vx = _packed(x)
+    vo = _packed_flat(out, (k,))
     idx = cnt = None
     vi = vc = None
     if want_aux:
         idx = Storage.allocate(k, Dtype.Int64, Device.Cuda)
         cnt = Storage.allocate(k, Dtype.Int32, Device.Cuda)
-        vi = flat_view(idx, (k,))
-        vc = flat_view(cnt, (k,))
+        vi = _packed_flat(idx, (k,))
+        vc = _packed_flat(cnt, (k,))
     arr = _lib.axes_array(axes)
-    _lib.call(
-        "nt_reduce", op, ctypes.byref(vx), arr, len(axes), ctypes.byref(vo), _lib.ref(vi), _lib.ref(vc)
-    )
+    _lib.call_packed("nt_reduce", op, vx, arr, len(axes), vo, vi, vc)
     if want_aux:
         return out, idx, cnt
     return out
@@ -252,9 +257,9 @@ def mean(x, axes, out_dtype: Dtype) -> Storage:
     require_device(x)
     k = _numel([s for i, s in enumerate(x._shape) if i not in axes])
     out = Storage.allocate(k, out_dtype, Device.Cuda)
-    vx = view_of(x)
-    vo = flat_view(out, (k,))
-    _lib.call("nt_mean", ctypes.byref(vx), _lib.axes_array(axes), len(axes), ctypes.byref(vo))
+    vx = _packed(x)
+    vo = _packed_flat(out, (k,))
+    _lib.call_packed("nt_mean", vx, _lib.axes_array(axes), len(axes), vo)
     return out
 
 
@@ -265,28 +270,28 @@ def reduce_bwd(op: int, g, scale: float, idx, cnt, axes, shape, target):
     require_device(g)
     g = g._to_contiguous()
     k = g.numel
-    vg = _lib.make_view(g._storage.data_ptr(), g._offset, int(g.dtype), (k,), (1,))
-    vi = flat_view(idx, (k,)) if idx is not None else None
-    vc = flat_view(cnt, (k,)) if cnt is not None else None
+    vg = _lib.pack_view(g._storage._ptr, g._offset, g._storage._dtype, (k,), (1,))
+    vi = _packed_flat(idx, (k,)) if idx is not None else None
+    vc = _packed_flat(cnt, (k,)) if cnt is not None else None
     arr = _lib.axes_array(axes)
     if target is None:
         out = Storage.allocate(_numel(shape), g.dtype, Device.Cuda)
-        vo = flat_view(out, shape)
+        vo = _packed_flat(out, shape)
         acc = 0
     else:
         out = None
-        vo = view_of(target)
+        vo = _packed(target)
         acc = 1
-    _lib.call(
+    _lib.call_packed(
         "nt_reduce_bwd",
         op,
-        ctypes.byref(vg),
+        vg,
         float(scale),
-        _lib.ref(vi),
-        _lib.ref(vc),
+        vi,
+        vc,
         arr,
         len(axes),
-        ctypes.byref(vo),
+        vo,
         acc,
     )
     if target is not None:
@@ -303,9 +308,9 @@ def matmul(x1, x2, out_shape) -> Storage:
     if x1.dtype != x2.dtype:
         raise RuntimeError("matmul: dtype mismatch")
     out = Storage.allocate(_numel(out_shape), x1.dtype, Device.Cuda)
-    v1, v2 = view_of(x1), view_of(x2)
-    vo = flat_view(out, out_shape)
-    _lib.call("nt_matmul", ctypes.byref(v1), ctypes.byref(v2), ctypes.byref(vo), 0)
+    v1, v2 = _packed(x1), _packed(x2)
+    vo = _packed_flat(out, out_shape)
+    _lib.call_packed("nt_matmul", v1, v2, vo, 0)
     return out
 
 
@@ -315,17 +320,16 @@ def matmul_bias(x1, x2, bias, out_shape) -> Storage:
     product followed by a broadcast add."""
     require_device(x1, x2, bias)
     out = Storage.allocate(_numel(out_shape), x1.dtype, Device.Cuda)
-    v1, v2, vb = view_of(x1), view_of(x2), view_of(bias)
-    vo = flat_view(out, out_shape)
-    _lib.call("nt_matmul_bias", ctypes.byref(v1), ctypes.byref(v2), ctypes.byref(vb),
-              ctypes.byref(vo))
+    v1, v2, vb = _packed(x1), _packed(x2), _packed(bias)
+    vo = _packed_flat(out, out_shape)
+    _lib.call_packed("nt_matmul_bias", v1, v2, vb, vo)
     return out
 
 
 def matmul_into(x1, x2, target, accumulate: bool) -> None:
     require_device(x1, x2, target)
-    v1, v2, vo = view_of(x1), view_of(x2), view_of(target)
-    _lib.call("nt_matmul", ctypes.byref(v1), ctypes.byref(v2), ctypes.byref(vo), int(accumulate))
+    v1, v2, vo = _packed(x1), _packed(x2), _packed(target)
+    _lib.call_packed("nt_matmul", v1, v2, vo, int(accumulate))
     target._storage.bump_version()
 
 

@@ -15,6 +15,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 from ctypes import POINTER, c_char_p, c_double, c_float, c_int, c_int32, c_int64
 from ctypes import c_size_t, c_uint64, c_void_p
 
@@ -103,6 +104,9 @@ _SIGNATURES = {
 }
 
 _lib: ctypes.CDLL | None = None
+# The entry points again, taking views as pack_view's bytes: packing one with
+# struct costs 0.7 us, filling an NtView field by field 3.
+_packed: dict = {}
 _load_error: str | None = None
 
 
@@ -129,6 +133,11 @@ def load() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
+        if _VP in args:
+            fn = lib[name]  # a function object of its own
+            fn.restype = res
+            fn.argtypes = [c_char_p if a is _VP else a for a in args]
+            _packed[name] = fn
     _lib = lib
     return lib
 
@@ -154,7 +163,31 @@ def check(rc: int) -> None:
 
 def call(name: str, *args) -> None:
     """Calls a status-returning entry point and raises on failure."""
-    check(getattr(load(), name)(*args))
+    rc = getattr(_lib or load(), name)(*args)
+    if rc != NT_OK:
+        check(rc)
+
+
+def call_packed(name: str, *args) -> None:
+    """`call` with every view given as pack_view's bytes (or None)."""
+    if _lib is None:
+        load()
+    rc = _packed[name](*args)
+    if rc != NT_OK:
+        check(rc)
+
+
+_pack = struct.Struct("=Qqii16q").pack
+_PAD = [(0,) * (NT_MAX_DIMS - n) for n in range(NT_MAX_DIMS + 1)]
+
+
+def pack_view(data: int, offset: int, dtype: int, shape, strides) -> bytes:
+    """The bytes of an NtView (same layout: no padding between its fields)."""
+    nd = len(shape)
+    if nd > NT_MAX_DIMS:
+        raise RuntimeError(f"Tensors are limited to {NT_MAX_DIMS} dims on device.")
+    pad = _PAD[nd]
+    return _pack(data, offset, dtype, nd, *shape, *pad, *strides, *pad)
 
 
 def is_available() -> bool:

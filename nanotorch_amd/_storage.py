@@ -20,8 +20,8 @@ class Storage:
     __slots__ = ("_dtype", "_device", "_size", "_ptr", "_host", "version", "__weakref__")
 
     def __init__(self, size: int, dtype: Dtype, device: Device, *, _zero: bool = True):
-        self._dtype = Dtype(dtype)
-        self._device = Device(device)
+        self._dtype = dtype if type(dtype) is Dtype else Dtype(dtype)
+        self._device = device if type(device) is Device else Device(device)
         self._size = int(size)
         self.version = 0
         self._ptr = None
@@ -30,7 +30,10 @@ class Storage:
             self._host = (ctype_of(self._dtype) * max(1, self._size))()
         else:
             p = ctypes.c_void_p()
-            _lib.call("nt_malloc", ctypes.byref(p), max(1, self._size) * sizeof(self._dtype))
+            lib = _lib._lib or _lib.load()
+            rc = lib.nt_malloc(ctypes.byref(p), (self._size or 1) * sizeof(self._dtype))
+            if rc:
+                _lib.check(rc)
             self._ptr = p.value
             if _zero and self._size > 0:
                 _lib.call("nt_fill", self._ptr, int(self._dtype), self._size, 0.0)

@@ -46,11 +46,11 @@ class Function:
         if self._saved_tensors is None:
             raise RuntimeError("No tensor was saved during forward.")
         for x, v in self._saved_tensors:
-            if x.version != v:
+            if x._storage.version != v:
                 raise RuntimeError(
                     "One of the tensors needed for grad computation was modified inplace."
                 )
-        return tuple(x for x, _ in self._saved_tensors)
+        return tuple([x for x, _ in self._saved_tensors])
 
     @classmethod
     def apply(cls, *args: Any, **kwargs: Any) -> Tensor:
@@ -59,15 +59,20 @@ class Function:
         self._inputs_kw = kwargs
         output = self.forward(*args, **kwargs)
         if is_grad_enabled():
-            if any(output is a for a in list(args) + list(kwargs.values())):
+            is_arg = tracked = False
+            for a in args:
+                if isinstance(a, Tensor):
+                    is_arg = is_arg or a is output
+                    tracked = tracked or a._requires_grad or a._grad_fn is not None
+            if is_arg or (kwargs and any(output is a for a in kwargs.values())):
                 output = output._alias()  # keeps the DAG structure
-            if any(isinstance(t, Tensor) and t.requires_grad for t in args):
+            if tracked:
                 output.attach_grad_fn(self)
         return output
 
     def save_for_backward(self, *tensors: Tensor) -> None:
         if is_grad_enabled():
-            self._saved_tensors = tuple((x, x.version) for x in tensors)
+            self._saved_tensors = tuple([(x, x._storage.version) for x in tensors])
 
     def fused_ok(self) -> bool:
         """Whether _backward_into handles this instance."""

@@ -18,9 +18,10 @@ import math
 
 from .. import _kernels as K
 from .. import _lib
-from .._data_type import is_float, promote_dtypes, sizeof
+from .._data_type import Dtype, is_float, promote_dtypes, sizeof
 from .._indexing import broadcast_shapes
-from ..core import Tensor, TensorShape
+from ..core import Tensor, TensorShape, expand_view, reshape_view, swap_last_view
+from ..cuda import Device
 from .function import Function
 from .grad_mode import is_grad_enabled
 from .ops_utils import unbroadcast
@@ -52,13 +53,12 @@ class _ElementwiseBinary(Function):
     def _backward_into(self, g: Tensor, needs, targets):
         op = self._op
         out_shape = self._out_shape
-        if g.shape != out_shape:
-            g = g.reshape(*out_shape)
+        g = reshape_view(g, out_shape)
         a = b = None
         if op in (_lib.MUL, _lib.DIV):
             x1, x2 = self.saved_tensors
-            a = x1.expand(*out_shape)
-            b = x2.expand(*out_shape)
+            a = expand_view(x1, out_shape)
+            b = expand_view(x2, out_shape)
         results = [None, None]
         # Gradients the kernel produces at full (output) shape.
         kneed = [False, False]
@@ -166,10 +166,10 @@ class MatmulOp(Function):
         self._shape1, self._shape2, shape_out = _matmul_broadcast(x1.shape, x2.shape)
         dtype = promote_dtypes(x1.dtype, x2.dtype)
         self._dtypes = (x1.dtype, x2.dtype, dtype)
-        x1 = x1.to(dtype).expand(*self._shape1)
+        x1 = expand_view(x1.to(dtype), self._shape1)
         if x2.ndim == 1 and self._shape2[-2:] == (x2.shape[0], 1):
-            x2 = x2.reshape(x2.shape[0], 1)  # cannot expand to the right
-        x2 = x2.to(dtype).expand(*self._shape2)
+            x2 = reshape_view(x2, (x2.shape[0], 1))  # cannot expand to the right
+        x2 = expand_view(x2.to(dtype), self._shape2)
         full_out = tuple(self._shape1[:-2]) + (self._shape1[-2], self._shape2[-1])
         st = K.matmul(x1, x2, full_out)
         return Tensor._new_contiguous(st, shape_out)
@@ -211,11 +211,10 @@ class MatmulOp(Function):
         the product's epilogue."""
         x1, x2 = self.saved_tensors
         full_out = tuple(self._shape1[:-2]) + (self._shape1[-2], self._shape2[-1])
-        if g.shape != full_out:
-            g = g.reshape(*full_out)
+        g = reshape_view(g, full_out)
         results = [None, None]
         if needs[0]:
-            rhs = x2.transpose(-2, -1)
+            rhs = swap_last_view(x2)
             if targets[0] is None:
                 st = K.matmul(g, rhs, x1.shape)
                 results[0] = Tensor._new_contiguous(st, x1.shape)
@@ -223,7 +222,7 @@ class MatmulOp(Function):
                 K.matmul_into(g, rhs, targets[0], accumulate=True)
                 results[0] = targets[0]
         if needs[1]:
-            lhs = x1.transpose(-2, -1)
+            lhs = swap_last_view(x1)
             if targets[1] is None:
                 st = K.matmul(lhs, g, x2.shape)
                 results[1] = Tensor._new_contiguous(st, x2.shape)
@@ -271,8 +270,8 @@ class LinearOp(Function):
     def _backward_into(self, g: Tensor, needs, targets):
         x, W = self.saved_tensors
         results = [None, None, None]
-        for i, (lhs, rhs, shape) in enumerate(((g, W.transpose(0, 1), x.shape),
-                                               (x.transpose(0, 1), g, W.shape))):
+        for i, (lhs, rhs, shape) in enumerate(((g, swap_last_view(W), x.shape),
+                                               (swap_last_view(x), g, W.shape))):
             if not needs[i]:
                 continue
             if targets[i] is None:
@@ -293,8 +292,6 @@ class LinearOp(Function):
     def usable(cls, x: Tensor, W: Tensor, b: Tensor) -> bool:
         """Whether the fused form applies: 2-D float32 x and W and a 1-D
         float32 b over W's columns, all on the device."""
-        from .._data_type import Dtype
-        from ..cuda import Device
         return (x.ndim == 2 and W.ndim == 2 and b.ndim == 1 and b.shape[0] == W.shape[1]
                 and x.shape[1] == W.shape[0]
                 and all(t.device == Device.Cuda and t.dtype == Dtype.Float32 for t in (x, W, b)))
@@ -314,11 +311,13 @@ def _binary_kernel_op(x1: Tensor, x2: Tensor, op: int, out: Tensor | None = None
     else:
         dtype = promote_dtypes(x1.dtype, x2.dtype)
         shape = broadcast_shapes(x1.shape, x2.shape)
+    if out is None:
+        x1 = expand_view(x1.to(dtype), shape)
+        x2 = expand_view(x2.to(dtype), shape)
+        return Tensor._new_contiguous(K.binary(op, x1, x2), shape)
     out_is_x1 = out is x1
     x1 = x1.to(dtype).expand(*shape)
     x2 = x2.to(dtype).expand(*shape)
-    if out is None:
-        return Tensor._new_contiguous(K.binary(op, x1, x2), shape)
     if out_is_x1:
         K.inplace(op, x1, x2)
         return x1

@@ -25,7 +25,7 @@ from .. import _kernels as K
 from .. import _lib
 from .._data_type import Dtype, is_float, sizeof
 from .._indexing import TensorShape
-from ..core import Tensor
+from ..core import Tensor, expand_view, reshape_view
 from ..cuda import Device
 from .function import Function
 from .ops_utils import broadcast_axis
@@ -75,7 +75,10 @@ class SumOp(Function):
     def _backward_into(self, g: Tensor, needs, targets):
         if not needs[0]:
             return [None]
-        (view,) = self.backward(g)
+        view = g
+        if self._orig_shape:
+            kd = _keepdim_shape(self._orig_shape, self._axis)
+            view = expand_view(reshape_view(g, kd), self._orig_shape)
         if targets[0] is None:
             return [view]
         K.inplace(_lib.ADD, targets[0], view)

@@ -5,7 +5,7 @@ from __future__ import annotations
 
 import math
 
-from ..core import Tensor
+from ..core import Tensor, expand_view
 from .function import Function
 from .ops_utils import unbroadcast
 
@@ -31,24 +31,8 @@ class ExpandOp(Function):
     are prepended)."""
 
     def forward(self, x: Tensor, *dims: int) -> Tensor:
-        if len(dims) < x.ndim:
-            raise ValueError(f"Cannot broadcast {x.shape} to {dims}.")
         self._orig_shape = x.shape
-        if dims == x.shape:
-            return x
-        strides = list(x._strides)
-        for i in range(len(dims)):
-            if i >= x.ndim:
-                strides = [0] + strides
-            else:
-                src, tgt = x.shape[-i - 1], dims[-i - 1]
-                if src == tgt:
-                    continue
-                if src == 1:
-                    strides[-i - 1] = 0
-                else:
-                    raise ValueError(f"Cannot broadcast {x.shape} to {dims} (mismatch).")
-        return Tensor._new_view(x.storage, tuple(dims), tuple(strides), x._offset)
+        return expand_view(x, dims)
 
     def backward(self, grad_out: Tensor) -> tuple[Tensor]:
         return (unbroadcast(grad_out, self._orig_shape),)

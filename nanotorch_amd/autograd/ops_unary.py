@@ -12,7 +12,7 @@ from __future__ import annotations
 from .. import _kernels as K
 from .. import _lib
 from .._data_type import Dtype, is_float, promote_dtypes, sizeof
-from ..core import Tensor
+from ..core import Tensor, reshape_view
 from .function import Function
 from .ops_utils import unbroadcast
 
@@ -61,8 +61,7 @@ class _UnaryOp(Function):
         if not needs[0]:
             return [None]
         saved = self._fused_saved()
-        if g.shape != saved.shape and saved is not None:
-            g = g.reshape(*saved.shape)
+        g = reshape_view(g, saved._shape)
         st = K.unary_bwd(self._op, g, saved, self._scalar(), targets[0])
         if st is None:
             return [targets[0]]
@@ -94,8 +93,7 @@ class NegOp(_UnaryOp):
     def _backward_into(self, g: Tensor, needs, targets):
         if not needs[0]:
             return [None]
-        if g.shape != self._shape:
-            g = g.reshape(*self._shape)
+        g = reshape_view(g, self._shape)
         st = K.unary_bwd(_lib.NEG, g, None, 0.0, targets[0])
         if st is None:
             return [targets[0]]
@@ -204,7 +202,10 @@ class PowOp(Function):
         if not isinstance(exponent, Tensor):
             exponent = Tensor(exponent)
         dtype = promote_dtypes(x.dtype, exponent.dtype)
-        e = float(exponent.cpu().item())
+        e = getattr(exponent, "_host_value", None)
+        if e is None or exponent.version != 0:
+            e = exponent.cpu().item()
+        e = float(e)
         if e < 0 and dtype <= Dtype.Int64:
             raise RuntimeError("Cannot use negative exponent with integer tensor.")
         self._x_dtype = x.dtype

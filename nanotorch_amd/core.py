@@ -28,7 +28,7 @@ from ._data_type import (
     promote_dtypes,
     sizeof,
 )
-from ._indexing import TensorShape, expand_ellipsis, is_contiguous_view
+from ._indexing import TensorShape, expand_ellipsis, is_contiguous_view, row_major_strides
 from ._storage import Storage
 from .cuda import Device, DeviceLiteral, get_std_device
 
@@ -94,7 +94,13 @@ class Tensor:
 
     @classmethod
     def _new_contiguous(cls, storage: Storage, shape: TensorShape) -> Tensor:
-        return cls._new_view(storage, tuple(shape), None, None)
+        shape = tuple(shape)
+        n = math.prod(shape)
+        if n > storage._size:
+            raise IndexError(
+                f"View max index {n - 1} exceeds storage capacity {storage.size}."
+            )
+        return cls._unchecked_view(storage, shape, row_major_strides(shape), 0)
 
     @classmethod
     def _new_view(
@@ -114,6 +120,13 @@ class Tensor:
                 raise IndexError(
                     f"View max index {hi} exceeds storage capacity {storage.size}."
                 )
+        return cls._unchecked_view(storage, shape, strides, offset)
+
+    @classmethod
+    def _unchecked_view(
+        cls, storage: Storage, shape: TensorShape, strides: TensorShape, offset: int
+    ) -> Tensor:
+        """A view known to lie within its storage (tuples given)."""
         new = cls.__new__(cls)
         new._storage = storage
         new._shape = shape
@@ -431,7 +444,7 @@ class Tensor:
         return Tensor._new_contiguous(K.clone_contiguous(self), self._shape)
 
     def _alias(self) -> Tensor:
-        return Tensor._new_view(self._storage, self._shape, self._strides, self._offset)
+        return Tensor._unchecked_view(self._storage, self._shape, self._strides, self._offset)
 
 
 # ------------------------------------------------------------------ helpers
@@ -498,13 +511,48 @@ def _from_array_like(data, user_dtype, device):
     return Storage.from_buffer(arr, dt, device), shape, dt
 
 
-def _infer_strides(shape: TensorShape) -> TensorShape:
-    strides = []
-    acc = 1
-    for s in reversed(shape):
-        strides.append(acc)
-        acc *= s
-    return tuple(reversed(strides))
+_infer_strides = row_major_strides
+
+
+# The views below are what the ops compute with, without a graph node: the
+# op that made them records its own.
+
+
+def expand_view(x: Tensor, dims: TensorShape) -> Tensor:
+    """x broadcast to `dims` by stride-0 axes; x itself if nothing changes."""
+    shape = x._shape
+    if dims == shape:
+        return x
+    lead = len(dims) - len(shape)
+    if lead < 0:
+        raise ValueError(f"Cannot broadcast {shape} to {dims}.")
+    strides = [0] * lead
+    for src, st, tgt in zip(shape, x._strides, dims[lead:]):
+        if src != tgt:
+            if src != 1:
+                raise ValueError(f"Cannot broadcast {shape} to {dims} (mismatch).")
+            st = 0
+        strides.append(st)
+    if 0 in shape or any(d < 0 for d in dims):
+        return Tensor._new_view(x._storage, dims, tuple(strides), x._offset)
+    return Tensor._unchecked_view(x._storage, dims, tuple(strides), x._offset)
+
+
+def reshape_view(x: Tensor, dims: TensorShape) -> Tensor:
+    """x with shape `dims` (of as many elements), copied first unless it is
+    contiguous; x itself if nothing changes."""
+    if dims == x._shape:
+        return x
+    x = x._to_contiguous()
+    return Tensor._new_view(x._storage, dims, None, x._offset)
+
+
+def swap_last_view(x: Tensor) -> Tensor:
+    """x with its last two axes swapped."""
+    shape, st = x._shape, x._strides
+    return Tensor._unchecked_view(
+        x._storage, shape[:-2] + (shape[-1], shape[-2]), st[:-2] + (st[-1], st[-2]), x._offset
+    )
 
 
 def _str_list_compact(li: Any) -> str:
@@ -569,30 +617,30 @@ def _backpropagate_grad(seed: Tensor) -> None:
     order: list[tuple[Tensor, Any, tuple]] = []
     while to_visit:
         f_x = to_visit.pop(0)
-        fn = f_x.grad_fn
+        fn = f_x._grad_fn
         if fn is None:
             continue
         inputs = []
         for x in fn.inputs:
             if isinstance(x, Tensor):
-                if x.requires_grad:
+                if x._requires_grad or x._grad_fn is not None:
                     ncons[id(x)] = ncons.get(id(x), 0) + 1
                     to_visit.append(x)
                 inputs.append(x)
         order.append((f_x, fn, tuple(inputs)))
 
     for f_x, fn, inputs in order:
-        if f_x.grad is None:
+        if f_x._grad is None:
             raise RuntimeError("f_x.grad is None.")
         ncons[id(f_x)] -= 1
         if ncons[id(f_x)] > 0:
             continue
-        _run_backward(fn, f_x.grad, inputs)
+        _run_backward(fn, f_x._grad, inputs)
         f_x._grad = None
 
 
 def _has_overlap(t: Tensor) -> bool:
-    return any(st == 0 and s > 1 for s, st in zip(t._shape, t._strides))
+    return 0 in t._strides and any(st == 0 and s > 1 for s, st in zip(t._shape, t._strides))
 
 
 def _accumulation_target(x: Tensor) -> Tensor | None:
@@ -620,20 +668,21 @@ def _store_first(x: Tensor, r: Tensor, upstream: Tensor) -> None:
 
 
 def _run_backward(fn, grad: Tensor, inputs: tuple) -> None:
-    needs = [x.requires_grad for x in inputs]
+    needs = [x._requires_grad or x._grad_fn is not None for x in inputs]
     fused = getattr(fn, "_backward_into", None)
-    distinct = len({id(x) for x in inputs}) == len(inputs)
     if fused is not None and fused.__self__.fused_ok():
-        if distinct:
-            groups = [list(range(len(inputs)))]
+        if len(inputs) == 1 or len({id(x) for x in inputs}) == len(inputs):
+            groups = None  # all inputs at once
         else:
             # The same tensor feeds several inputs (e.g. x * x): hand out the
             # gradients one input at a time so each lands on the value the
             # previous one left, as `x._grad = g; x._grad += g2` does.
             groups = [[i] for i in range(len(inputs))]
-        for grp in groups:
-            sub_needs = [needs[i] and i in grp for i in range(len(inputs))]
-            if not any(sub_needs):
+        for grp in groups or (None,):
+            sub_needs = needs if grp is None else [
+                needs[i] and i in grp for i in range(len(inputs))
+            ]
+            if True not in sub_needs:
                 continue
             targets = [
                 _accumulation_target(x) if n else None

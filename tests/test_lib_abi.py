@@ -61,3 +61,16 @@ def test_noalloc_entry_point_refuses_before_init():
     rc = lib.nt_reduce_noalloc(0, None, None, 0, None, None, None)
     assert rc == _lib.NT_ERR_RUNTIME
     assert b"nt_init" in lib.nt_last_error()
+
+
+def test_packed_view_has_the_bytes_of_a_view():
+    """pack_view is what the ops pass in place of an NtView."""
+    import ctypes
+
+    for shape, strides in (((), ()), ((3,), (2,)), ((4, 5), (0, 1)),
+                           (tuple(range(1, 9)), tuple(range(8)))):
+        v = _lib.make_view(0xFEDC00001000, 7, 3, shape, strides)
+        packed = _lib.pack_view(0xFEDC00001000, 7, 3, shape, strides)
+        assert packed == ctypes.string_at(ctypes.addressof(v), ctypes.sizeof(v))
+    with pytest.raises(RuntimeError):
+        _lib.pack_view(0x1000, 0, 3, (1,) * 9, (1,) * 9)
