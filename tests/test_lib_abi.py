@@ -7,6 +7,7 @@ import ctypes
 import os
 import re
 
+import pytest
 from conftest import ROOT
 
 from nanotorch_amd import _lib
@@ -65,8 +66,6 @@ def test_noalloc_entry_point_refuses_before_init():
 
 def test_packed_view_has_the_bytes_of_a_view():
     """pack_view is what the ops pass in place of an NtView."""
-    import ctypes
-
     for shape, strides in (((), ()), ((3,), (2,)), ((4, 5), (0, 1)),
                            (tuple(range(1, 9)), tuple(range(8)))):
         v = _lib.make_view(0xFEDC00001000, 7, 3, shape, strides)
