@@ -1,6 +1,8 @@
 // Batched matmul C[b] = A[b] . B[b] (+ C_old[b]) on strided views.
 //
-// fp32 runs on the gfx950 matrix cores (v_mfma_f32_32x32x2_f32).  The
+// fp32 runs on the gfx950 matrix cores (v_mfma_f32_32x32x2_f32; large single
+// products on v_mfma_f32_32x32x16_bf16 with each operand split into three
+// exact parts, see mm_split_kernel).  The
 // reference (src/cpp/ops/matmul.cu) has a SIMT 128x128x16 kernel that only
 // accepts contiguous operands and sends every transposed operand -- hence
 // both backward products of MatmulOp (ops_binary.py:264-267) -- to a naive
@@ -73,6 +75,10 @@ struct MMArgs {
   // would give); nullptr: none.  Never combined with accumulate.
   const float *bias;
   int64_t sBias;
+  // Flag words of a split product (mm_split_pack_kernel): the kernel runs
+  // only if they say `run_if`.  nullptr: it runs.
+  const uint32_t *flags;
+  bool run_if;
 };
 
 // Workgroup -> (slice of K, batch, tile).
@@ -305,6 +311,18 @@ __device__ __forceinline__ void dl_wait_and_sync() {
   __syncthreads();
 }
 
+constexpr uint32_t SP_BAD = 1, SP_SMALL = 2;
+
+// Flags of both operands of a split product (mm_split_pack_kernel): whether
+// it is within the range where the parts do what float32 does.  SP_BAD: a
+// value that is not finite, 2^50 or more, or non-zero below 2^-60; SP_SMALL: a
+// non-zero one below 2^-40.  Without SP_BAD, and with SP_SMALL in at most one
+// operand, every non-zero product is in [2^-100, 2^100]: the products of its
+// parts, down to 2^-24 of it, are normal, and 2^27 of them cannot overflow.
+__device__ __forceinline__ bool split_ok(const uint32_t *flags) {
+  return !((flags[0] | flags[1]) & SP_BAD) && !(flags[0] & flags[1] & SP_SMALL);
+}
+
 // A BM x BN tile of a slice of K: 4 waves in a WM x WN grid, each a
 // (BM / WM) x (BN / WN) block of 32x32 MFMA blocks.  Operands staged by
 // direct loads into two named stage pairs (the k loop is unrolled by two so
@@ -332,6 +350,8 @@ void mm_f32_tile_kernel(MMArgs g) {
   const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wm = wave / WN, wn = wave % WN;
   const int h = lane >> 5, li = lane & 31;
+  if (g.flags && split_ok(g.flags) != g.run_if)
+    return;
   const TileCoord tc = mm_tile_coord<BM, BN>(g);
 
   floatx16 acc[NM][NN];
@@ -651,6 +671,250 @@ __global__ __launch_bounds__(WD_THREADS, 1) void mm_f32_mfma_wide_kernel(
     }
 }
 
+// ------------------------------------- large products on the bf16 matrix cores
+
+// A float32 is the exact sum of three bfloat16 values (8 + 8 + 8 bits of
+// significand), and a product of bfloat16 values is exact in float32.  So
+// a . b = (a1 + a2 + a3) . (b1 + b2 + b3) can run on the bf16 MFMA, which does
+// 16 times the work of the fp32 one per cycle, accumulating in float32 as
+// before: six of the nine products, the three left out (a2 b3, a3 b2, a3 b3)
+// are below 2^-26 of a b, under the rounding of a float32 product.
+// Error against 64 bits (2-norm), fp32 MFMA -> this: normal operands 4096^3
+// 1.15e-6 -> 9.7e-7, 4096x1000x4096 5.7e-7 -> 4.8e-7, 4096x320x4096 3.2e-7 ->
+// 2.7e-7, 1024x8192x4096 8.1e-7 -> 6.9e-7; uniform [0, 1) 4096^3 8.4e-7 ->
+// 5.2e-7: 6 roundings of the sum per 16 k's where the fp32 MFMA has 8 and the
+// products' own.  Mean shift of the results: at most 7e-9 of their mean
+// magnitude (4e-9 before).
+//
+// Three kernels: mm_split_pack_kernel writes both operands as packed bf16
+// planes, in the order in which the product's LDS stages hold them, zeros
+// past every edge; mm_split_kernel multiplies; the slices of a split K are
+// added as for the other tiles.  What six exact products cannot do as the
+// fp32 kernel does -- infinities and NaN (0 x inf among the parts), parts or
+// products outside the normal range -- the pack kernel reports in a flag
+// word per operand: then mm_split_kernel returns at once and the fp32 tile
+// kernel, queued behind it, does the work; otherwise that one returns at once.
+constexpr int SP_B = 256, SP_K = 16;             // rows of a block, k of a step
+constexpr int SP_PLANE = SP_B * SP_K;            // bf16 values
+constexpr int SP_STEP = 3 * SP_PLANE * 2;        // bytes of a block's k step
+// The bf16 MFMA rounds its sums down (towards -infinity): left alone, results
+// are 2.6e-7 of their mean magnitude too low, which does not average out in
+// what sums them next (a loss, a bias gradient).  So A's values are packed
+// negated in half of the runs of SP_FLIP steps, and the sums are negated where
+// the sign changes: down is then up, and the shifts cancel.  The signs follow
+// the parity of the run number's bits (+ - - + - + + -), which cancels the
+// growth of the sums, and of their roundings, along K as well.
+constexpr uint32_t SP_FLIP = 6; // a multiple of the k loop's 3
+__device__ __forceinline__ bool split_negated(uint32_t step) {
+  return __popc(step / SP_FLIP) & 1;
+}
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+__global__ void mm_split_flags_kernel(uint32_t *flags) {
+  if (threadIdx.x < 2)
+    flags[threadIdx.x] = 0;
+}
+
+struct SplitOperand {
+  const float *p;
+  int64_t rows, s_mn, s_k;
+  char *packed;
+  uint32_t blocks; // workgroups for this operand
+  int vec;         // k unit-stride, 16-byte aligned
+};
+
+// A wave packs 32 rows of one k step: lane l the 8 k's of half l / 32 of row
+// l % 32, 16 bytes in each plane, so that a wave writes 1 KB runs.  Packed
+// order: [256-row block][k step][plane][32-row block][half][row][8].  The 4
+// waves of a workgroup take consecutive k steps (64 k's: 256 bytes of a
+// k-contiguous row).  HBM bound: 4 bytes read, 6 written per value.
+__global__ __launch_bounds__(256) void mm_split_pack_kernel(
+    SplitOperand a, SplitOperand b, int64_t K, uint32_t ksteps, uint32_t *flags) {
+  const bool second = blockIdx.x >= a.blocks;
+  const SplitOperand &o = second ? b : a;
+  const uint32_t w = blockIdx.x - (second ? a.blocks : 0);
+  const uint32_t kgroups = (ksteps + 3) / 4;
+  const uint32_t rb = w / kgroups; // 32-row block
+  const int lane = threadIdx.x & 63;
+  const uint32_t step = (w - rb * kgroups) * 4 + (threadIdx.x >> 6);
+  if (step >= ksteps)
+    return;
+  const int64_t row = int64_t(rb) * 32 + lane % 32;
+  const int64_t k = int64_t(step) * SP_K + lane / 32 * 8;
+  float v[8];
+  if (o.vec && row < o.rows && k + 8 <= K) {
+    const float4 *q = reinterpret_cast<const float4 *>(o.p + row * o.s_mn + k);
+    const float4 x = q[0], y = q[1];
+    v[0] = x.x, v[1] = x.y, v[2] = x.z, v[3] = x.w;
+    v[4] = y.x, v[5] = y.y, v[6] = y.z, v[7] = y.w;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      v[e] = 0.f;
+      if (row < o.rows && k + e < K)
+        v[e] = o.p[row * o.s_mn + (k + e) * o.s_k];
+    }
+  }
+  bf16x8 p1, p2, p3;
+  uint32_t f = 0;
+  const bool neg = !second && split_negated(step);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t ex = (__float_as_uint(v[e]) >> 23) & 255; // 127: 1.x
+    const bool zero = v[e] == 0.f;
+    f |= ex >= 127 + 50 || (!zero && ex < 127 - 60) ? SP_BAD : 0;
+    f |= !zero && ex < 127 - 40 ? SP_SMALL : 0;
+    const float x = neg ? -v[e] : v[e];
+    p1[e] = __bf16(x);
+    const float r = x - float(p1[e]);
+    p2[e] = __bf16(r);
+    p3[e] = __bf16(r - float(p2[e]));
+  }
+  char *dst = o.packed + (int64_t(rb / 8) * ksteps + step) * SP_STEP +
+              (rb % 8) * (32 * SP_K * 2) + lane * 16;
+  *reinterpret_cast<bf16x8 *>(dst) = p1;
+  *reinterpret_cast<bf16x8 *>(dst + 2 * SP_PLANE) = p2;
+  *reinterpret_cast<bf16x8 *>(dst + 4 * SP_PLANE) = p3;
+  if (f) // rare: no traffic on the word for ordinary data
+    atomicOr(flags + second, f);
+}
+
+// 256x256 tiles, 8 waves in a 2x4 grid (two per SIMD) of 128x64: 4x2 blocks
+// of 32x32, 48 MFMAs of 32x32x16 per k step against 18 fragment reads, so
+// the matrix pipe, not LDS, is the bound.  Stages are copies of the packed
+// operands (every load 1 KB of consecutive memory, conflict-free reads).
+// Three stages keep the matrix pipe busy 84% of cycles (two: 75%), at which
+// the chip's power, not the kernel, sets the rate: the clock falls to 1.8 GHz.
+// 8192x4096x4096 with packing: 1930 us on the fp32 MFMA, 1200 here (229
+// TFLOP/s; 1232 with two stages); 4000^3 1062 -> 611 us, 8192x4096x1000 in two
+// slices of K 553 -> 368, 4096x300x4096 106 -> 71.
+__global__ __launch_bounds__(512, 1) void mm_split_kernel(
+    MMArgs g, const char *pa, const char *pb, uint32_t ksteps, uint32_t kper,
+    const uint32_t *flags) {
+  if (!split_ok(flags))
+    return;
+  __shared__ __align__(16) char sA0[SP_STEP], sB0[SP_STEP];
+  __shared__ __align__(16) char sA1[SP_STEP], sB1[SP_STEP];
+  __shared__ __align__(16) char sA2[SP_STEP], sB2[SP_STEP];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 2, wn = wave & 3;
+  const TileCoord tc = mm_tile_coord<SP_B, SP_B>(g);
+  floatx16 acc[4][2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        acc[i][j][r] = 0.f;
+  const uint32_t s0 = tc.slice * kper;
+  const uint32_t steps = ksteps - s0 < kper ? ksteps - s0 : kper;
+  const char *a0 = pa + (tc.m0 / SP_B * ksteps + s0) * SP_STEP;
+  const char *b0 = pb + (tc.n0 / SP_B * ksteps + s0) * SP_STEP;
+  auto issue = [&](char *sa, char *sb, uint32_t s) {
+    // a wave copies 3 KB of each operand's 24
+    auto copy = [&](char *stage, const char *src) {
+      const uint64_t ub = reinterpret_cast<uint64_t>(src + int64_t(s) * SP_STEP);
+      const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(ub));
+      const uint32_t hi = __builtin_amdgcn_readfirstlane(uint32_t(ub >> 32));
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+          reinterpret_cast<void *>((uint64_t(hi) << 32) | lo), 0, SP_STEP, BUF_WORD3);
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            rs,
+            (__attribute__((address_space(3))) void *)(stage + (wave * 3 + j) * 1024),
+            16, (wave * 3 + j) * 1024 + lane * 16, 0, 0, 0);
+    };
+    copy(sa, a0);
+    copy(sb, b0);
+  };
+  auto compute = [&](const char *sa, const char *sb) {
+    bf16x8 a[4][3], b[2][3];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        a[i][p] = *reinterpret_cast<const bf16x8 *>(sa + p * 2 * SP_PLANE +
+                                                    (wm * 4 + i) * 1024 + lane * 16);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        b[j][p] = *reinterpret_cast<const bf16x8 *>(sb + p * 2 * SP_PLANE +
+                                                    (wn * 2 + j) * 1024 + lane * 16);
+    }
+    // small products first
+    constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int q = 0; q < 6; ++q)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              a[i][PA[q]], b[j][PB[q]], acc[i][j], 0, 0, 0);
+  };
+  // Three stages: a step's loads have two steps of MFMAs to land in, so the
+  // wait leaves the 6 loads of the step after next in flight.  Past the end
+  // the last step is loaded again, to keep the count.  steps is a multiple
+  // of 3: one exit, so that the accumulators stay where they are.
+  auto landed = [] {
+    asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  auto at = [&](uint32_t s) { return s < steps ? s : steps - 1; };
+  issue(sA0, sB0, 0);
+  issue(sA1, sB1, 1);
+  landed();
+  auto negate = [&] {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          acc[i][j][r] = -acc[i][j][r];
+  };
+  for (uint32_t s = 0; s < steps; s += 3) {
+    if (s > 0 && split_negated(s0 + s) != split_negated(s0 + s - 1))
+      negate();
+    issue(sA2, sB2, s + 2);
+    pin_issued_loads();
+    compute(sA0, sB0);
+    landed();
+    issue(sA0, sB0, at(s + 3));
+    pin_issued_loads();
+    compute(sA1, sB1);
+    landed();
+    issue(sA1, sB1, at(s + 4));
+    pin_issued_loads();
+    compute(sA2, sB2);
+    landed();
+  }
+  if (split_negated(s0 + steps - 1))
+    negate();
+  // no load may still write the LDS of a workgroup that has ended
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  const int h = lane >> 5, li = lane & 31;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int64_t col = tc.n0 + wn * 64 + j * 32 + li;
+      if (col >= g.N)
+        continue;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int64_t row =
+            tc.m0 + wm * 128 + i * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
+        if (row < g.M)
+          mm_put(g, tc, row, col, acc[i][j][r]);
+      }
+    }
+}
+
 // C[b][m][n] (+)= part[0][b][m][n] + part[1][b][m][n] + ... in slice order (a
 // fixed order: the result does not depend on scheduling).  V adjacent columns
 // per work-item; V == 4 needs N a multiple of 4 and 16-byte rows of C.
@@ -660,7 +924,7 @@ __global__ __launch_bounds__(256) void mm_splitk_sum_kernel(
   // one work-item per V columns of one row, in a one-shot grid; the S slice
   // loads are independent (S is a template argument) and go out together
   const uint32_t q = blockIdx.x * 256u + threadIdx.x;
-  if (q >= total)
+  if (q >= total || (g.flags && split_ok(g.flags) != g.run_if))
     return;
   const uint32_t rm = fdn.div(q); // batch * M + m
   const int64_t n = int64_t(q - rm * fdn.d) * V;
@@ -862,6 +1126,43 @@ bool aligned16(const void *p) {
   return reinterpret_cast<uintptr_t>(p) % 16 == 0;
 }
 
+// Adds the S slices in a.part into C.
+void launch_sum(const MMArgs &a, int S) {
+  const int64_t outs = int64_t(a.nbatch) * a.M * a.N;
+  bool vec = a.N % 4 == 0 && a.sCn == 1 && a.sCm % 4 == 0 && aligned16(a.C);
+  for (int d = 0; d < a.nb; ++d)
+    vec = vec && a.bsC[d] % 4 == 0;
+  const FastDivU32 fdn{uint32_t(vec ? a.N / 4 : a.N)}, fdm{uint32_t(a.M)};
+  const int64_t items = vec ? outs / 4 : outs;
+  const dim3 grid{unsigned(ceil_div(items, 256)), 1u, 1u};
+  auto sum = [&]<int SS>() {
+    if (vec)
+      mm_splitk_sum_kernel<SS, 4>
+          <<<grid, 256, 0, stream()>>>(a, fdn, fdm, uint32_t(items));
+    else
+      mm_splitk_sum_kernel<SS, 1>
+          <<<grid, 256, 0, stream()>>>(a, fdn, fdm, uint32_t(items));
+  };
+  switch (S) {
+  case 2:
+    return sum.template operator()<2>();
+  case 3:
+    return sum.template operator()<3>();
+  case 4:
+    return sum.template operator()<4>();
+  case 6:
+    return sum.template operator()<6>();
+  case 8:
+    return sum.template operator()<8>();
+  case 12:
+    return sum.template operator()<12>();
+  case 16:
+    return sum.template operator()<16>();
+  default:
+    fail(NT_ERR_RUNTIME, "matmul: no split-K sum for this slice count");
+  }
+}
+
 // Runs `launch(args)` over S slices of K (each kslice long) into scratch and
 // adds them up; over one slice straight into C.  A split that the device
 // memory has no room for is not made.
@@ -891,38 +1192,7 @@ template <class F> void run_split(const MMArgs &a, int S, int64_t kslice, F laun
   w.part = static_cast<float *>(part);
   launch(w, S);
   NT_LAUNCH_CHECK();
-  bool vec = a.N % 4 == 0 && a.sCn == 1 && a.sCm % 4 == 0 && aligned16(a.C);
-  for (int d = 0; d < a.nb; ++d)
-    vec = vec && a.bsC[d] % 4 == 0;
-  const FastDivU32 fdn{uint32_t(vec ? a.N / 4 : a.N)}, fdm{uint32_t(a.M)};
-  const int64_t items = vec ? outs / 4 : outs;
-  const dim3 grid{unsigned(ceil_div(items, 256)), 1u, 1u};
-  auto sum = [&]<int SS>() {
-    if (vec)
-      mm_splitk_sum_kernel<SS, 4>
-          <<<grid, 256, 0, stream()>>>(w, fdn, fdm, uint32_t(items));
-    else
-      mm_splitk_sum_kernel<SS, 1>
-          <<<grid, 256, 0, stream()>>>(w, fdn, fdm, uint32_t(items));
-  };
-  switch (S) {
-  case 2:
-    return sum.template operator()<2>();
-  case 3:
-    return sum.template operator()<3>();
-  case 4:
-    return sum.template operator()<4>();
-  case 6:
-    return sum.template operator()<6>();
-  case 8:
-    return sum.template operator()<8>();
-  case 12:
-    return sum.template operator()<12>();
-  case 16:
-    return sum.template operator()<16>();
-  default:
-    fail(NT_ERR_RUNTIME, "matmul: no split-K sum for this slice count");
-  }
+  launch_sum(w, S);
 }
 
 // Tile shape and slices of K of mm_f32_tile_kernel for one product: the
@@ -940,6 +1210,7 @@ template <class F> void run_split(const MMArgs &a, int S, int64_t kslice, F laun
 struct TileChoice {
   int bm, bn, S;
   int64_t kslice;
+  double us; // the estimate
 };
 
 TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int64_t nbatch) {
@@ -961,7 +1232,7 @@ TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int64_t nbatch) {
     sum[i] = S == 1 ? 0 : SUM + (S + 1) * outs * (sizeof(float) / SUM_BYTES);
   }
   static constexpr int SHAPES[][2] = {{128, 128}, {64, 64}, {32, 128}, {128, 32}};
-  TileChoice best{128, 128, 1, K};
+  TileChoice best{128, 128, 1, K, 0};
   double best_t = std::numeric_limits<double>::infinity();
   for (const auto &sh : SHAPES) {
     const int bm = sh[0], bn = sh[1];
@@ -979,7 +1250,7 @@ TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int64_t nbatch) {
           double(kts[i]) * std::max(mfma, lat) + double(per_cu) * EPI * area + sum[i];
       if (t < best_t) {
         best_t = t;
-        best = {bm, bn, SPLITS[i], i == 0 ? K : kts[i] * MM_BK};
+        best = {bm, bn, SPLITS[i], i == 0 ? K : kts[i] * MM_BK, t};
       }
     }
   }
@@ -1000,7 +1271,9 @@ void launch_tile(const MMArgs &a, const TileChoice &c) {
 }
 
 template <int SA, int SB> void launch_stages(const MMArgs &a) {
-  const TileChoice c = choose_tile(a.M, a.N, a.K, a.nbatch);
+  // (as the fallback of a split product: rarely run, so unsplit)
+  const TileChoice c = a.flags ? TileChoice{128, 128, 1, a.K, 0}
+                               : choose_tile(a.M, a.N, a.K, a.nbatch);
   if (c.bm == 64)
     launch_tile<SA, SB, 64, 64>(a, c);
   else if (c.bm == 32)
@@ -1051,6 +1324,86 @@ template <int LA, int LB> bool launch_wide(const MMArgs &a) {
   return true;
 }
 
+// The product through packed bf16 planes (mm_split_kernel), where that is
+// estimated to take less than 0.92 of the fp32 time f32_us; false: not taken.
+// A k step of a tile takes 1.5 us with few CUs at work and 2.1 with all (the
+// clock falls with the power), packing 10 bytes per value at 5 TB/s and the
+// three small launches 12 us; measured against the estimate: 4000^3 611 us /
+// 616, 8192x4096x1000 368 / 390, 1024x8192x4096 388 / 396, 4096x300x4096
+// 71 / 69.  ak, bk: the operand has 16-byte aligned rows along k.
+template <class FB>
+bool launch_split(const MMArgs &a, double f32_us, bool ak, bool bk, FB fallback) {
+  if (f32_us < 40 || a.K >= (int64_t(1) << 27))
+    return false;
+  const int64_t tm = ceil_div(a.M, SP_B), tn = ceil_div(a.N, SP_B);
+  const int64_t ksteps = ceil_div(a.K, 3 * SP_K) * 3; // in threes, see the kernel
+  const int64_t cus = device_cu_count();
+  const double outs = double(a.M) * double(a.N);
+  double best_t = std::numeric_limits<double>::infinity();
+  int S = 1;
+  for (int s : {1, 2, 3, 4, 6, 8}) {
+    const int64_t per = ceil_div(ksteps, 3 * s) * 3;
+    if (ceil_div(ksteps, per) != s)
+      continue;
+    const double busy = std::min(1.0, double(tm * tn * s) / double(cus));
+    double t = double(ceil_div(tm * tn * s, cus)) * (double(per) * (1.5 + 0.6 * busy) + 8);
+    if (s > 1)
+      t += 4 + (s + 1) * outs * 4 / 6e6;
+    if (t < best_t) {
+      best_t = t;
+      S = s;
+    }
+  }
+  const double pack = 12 + double(tm + tn) * SP_B * double(a.K) * 10 / 5e6;
+  if (best_t + pack > 0.92 * f32_us)
+    return false;
+  const size_t abytes = size_t(tm * ksteps) * SP_STEP, bbytes = size_t(tn * ksteps) * SP_STEP;
+  const size_t pbytes = S > 1 ? size_t(S) * size_t(outs) * sizeof(float) : 0;
+  if (outs >= 4294967296. || tm * tn * S >= (int64_t(1) << 31) ||
+      (tm + tn) * 8 * ceil_div(ksteps, 4) >= (int64_t(1) << 31))
+    return false;
+  void *scratch = nullptr;
+  try {
+    scratch = device_alloc(256 + abytes + bbytes + pbytes);
+  } catch (const Error &e) {
+    if (e.code != NT_ERR_OOM)
+      throw;
+    return false;
+  }
+  struct Free {
+    void *p;
+    ~Free() { device_free(p); }
+  } owner{scratch};
+  uint32_t *flags = static_cast<uint32_t *>(scratch);
+  char *pa = static_cast<char *>(scratch) + 256, *pb = pa + abytes;
+  mm_split_flags_kernel<<<1, 64, 0, stream()>>>(flags);
+  NT_LAUNCH_CHECK();
+  const uint32_t kgroups = uint32_t(ceil_div(ksteps, 4));
+  const SplitOperand oa{a.A, a.M, a.sAm, a.sAk, pa, uint32_t(tm * 8) * kgroups, ak};
+  const SplitOperand ob{a.B, a.N, a.sBn, a.sBk, pb, uint32_t(tn * 8) * kgroups, bk};
+  mm_split_pack_kernel<<<oa.blocks + ob.blocks, 256, 0, stream()>>>(
+      oa, ob, a.K, uint32_t(ksteps), flags);
+  NT_LAUNCH_CHECK();
+  MMArgs w = a;
+  w.tiles_m = tm;
+  w.tiles_n = tn;
+  w.part = S > 1 ? reinterpret_cast<float *>(pb + bbytes) : nullptr;
+  mm_split_kernel<<<unsigned(tm * tn * S), 512, 0, stream()>>>(
+      w, pa, pb, uint32_t(ksteps), uint32_t(ceil_div(ksteps, 3 * S) * 3), flags);
+  NT_LAUNCH_CHECK();
+  w.flags = flags;
+  if (S > 1) {
+    w.run_if = true;
+    launch_sum(w, S);
+    NT_LAUNCH_CHECK();
+  }
+  w.part = nullptr;
+  w.run_if = false;
+  fallback(w);
+  NT_LAUNCH_CHECK();
+  return true;
+}
+
 // fp32 product; al: both operands' bases and batch strides are 16-byte
 // aligned.
 void launch_f32(const MMArgs &a, bool al) {
@@ -1063,13 +1416,38 @@ void launch_f32(const MMArgs &a, bool al) {
   const bool wide = (ak || am) && (bn || bk);
   const bool a_mn = wide ? !ak : a.sAm < a.sAk;
   const bool b_mn = wide ? bn : a.sBn < a.sBk;
+  constexpr int64_t FAR = int64_t(1) << 22;
+  const bool far = a.sAm > FAR || a.sAk > FAR || a.sBn > FAR || a.sBk > FAR;
+  auto tiles = [&](const MMArgs &g) {
+    if (wide) {
+      if (a_mn)
+        b_mn ? launch_stages<ST_MN16, ST_MN16>(g) : launch_stages<ST_MN16, ST_K16>(g);
+      else
+        b_mn ? launch_stages<ST_K16, ST_MN16>(g) : launch_stages<ST_K16, ST_K16>(g);
+    } else {
+      if (a_mn)
+        b_mn ? launch_stages<ST_MN4, ST_MN4>(g) : launch_stages<ST_MN4, ST_K4>(g);
+      else
+        b_mn ? launch_stages<ST_K4, ST_MN4>(g) : launch_stages<ST_K4, ST_K4>(g);
+    }
+  };
+  if (!far && a.nbatch == 1) {
+    // large tiles at 131 TFLOP/s, or the tile kernel's estimate (4-byte loads
+    // at 0.8 of its rate)
+    const double flops_us = 2. * double(a.M) * double(a.N) * double(a.K) / 131e6;
+    if (flops_us > 20) {
+      const double est = choose_tile(a.M, a.N, a.K, 1).us;
+      if (launch_split(a, wide ? std::max(flops_us, est) : 1.25 * std::max(flops_us, est),
+                       ak, bk, tiles))
+        return;
+    }
+  }
   if (wide && (a_mn ? (b_mn ? launch_wide<LAY_MN, LAY_MN>(a)
                             : launch_wide<LAY_MN, LAY_K>(a))
                     : (b_mn ? launch_wide<LAY_K, LAY_MN>(a)
                             : launch_wide<LAY_K, LAY_K>(a))))
     return;
-  constexpr int64_t FAR = int64_t(1) << 22;
-  if (a.sAm > FAR || a.sAk > FAR || a.sBn > FAR || a.sBk > FAR) {
+  if (far) {
     MMArgs w = a;
     w.kslice = a.K;
     w.tiles_m = ceil_div(a.M, 128);
@@ -1080,17 +1458,7 @@ void launch_f32(const MMArgs &a, bool al) {
     mm_f32_far_kernel<<<dim3(unsigned(blocks)), MM_THREADS, 0, stream()>>>(w);
     return;
   }
-  if (wide) {
-    if (a_mn)
-      b_mn ? launch_stages<ST_MN16, ST_MN16>(a) : launch_stages<ST_MN16, ST_K16>(a);
-    else
-      b_mn ? launch_stages<ST_K16, ST_MN16>(a) : launch_stages<ST_K16, ST_K16>(a);
-  } else {
-    if (a_mn)
-      b_mn ? launch_stages<ST_MN4, ST_MN4>(a) : launch_stages<ST_MN4, ST_K4>(a);
-    else
-      b_mn ? launch_stages<ST_K4, ST_MN4>(a) : launch_stages<ST_K4, ST_K4>(a);
-  }
+  tiles(a);
 }
 
 } // namespace

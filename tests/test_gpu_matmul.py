@@ -390,3 +390,83 @@ def test_other_dtypes_exact_in_every_tile(gpu, M, K_, N, layout, dt):
     if M < 100:
         got = _mm(xa.reshape(1, M, K_).expand(3, M, K_), xb.reshape(1, K_, N).expand(3, K_, N))
         assert_bitexact(got, np.broadcast_to(want, (3, M, N)), "batched")
+
+
+# --------------------------------------- large products on the bf16 planes
+
+def _cached_after(call):
+    """Bytes in the allocator's cache after `call` alone: its scratch."""
+    import ctypes
+
+    from nanotorch_amd import _lib
+    _lib.call("nt_empty_cache")
+    call()
+    nt.sync()
+    used, cached = ctypes.c_size_t(), ctypes.c_size_t()
+    _lib.call("nt_memory_stats", ctypes.byref(used), ctypes.byref(cached))
+    return cached.value
+
+
+# one slice and several of K; M, N and K off every tile, step and vector size
+SPLIT_SHAPES = [(4096, 320, 4096), (4093, 301, 4090), (1020, 8200, 4100), (2300, 4101, 2305)]
+
+
+@pytest.mark.parametrize("layout", ["NN", "TN", "NT", "TT"])
+@pytest.mark.parametrize("M,K_,N", SPLIT_SHAPES)
+def test_split_product(gpu, M, K_, N, layout):
+    """Products that run as three bf16 parts per operand: every output within
+    the bound of a float32 sum in any order (K 2^-24 (|A|.|B|)), and in
+    2-norm no further from 64 bits than 1.1 of sqrt(K) / 2 roundings."""
+    r = rng(seed_of("split", M, K_, N, layout))
+    a = r.standard_normal((M, K_), dtype=np.float32)
+    b = r.standard_normal((K_, N), dtype=np.float32) / np.float32(np.sqrt(K_))
+    xa = dev_T(a) if layout[0] == "T" else dev(a)
+    xb = dev_T(b) if layout[1] == "T" else dev(b)
+    old = r.standard_normal((M, N), dtype=np.float32)
+    tgt = dev(old)
+    packed = 6 * (M * K_ + K_ * N)
+    assert _cached_after(lambda: K.matmul_into(xa, xb, tgt, accumulate=False)) >= packed
+    want = a.astype(np.float64) @ b
+    scale = np.abs(a).astype(np.float64) @ np.abs(b)
+    got = host(tgt)
+    err = np.abs(got - want)
+    assert (err / scale).max() <= K_ * 2.0**-24
+    assert np.linalg.norm(err) <= 1.1 * np.sqrt(K_) / 2 * 2.0**-24 * np.linalg.norm(want) + 2.0**-24
+    tgt = dev(old)
+    K.matmul_into(xa, xb, tgt, accumulate=True)
+    assert_bitexact(host(tgt), old + got, "accumulated")
+
+
+@pytest.mark.parametrize("special", ["inf", "nan", "large", "tiny", "tiny row", "both small", "zeros"])
+@pytest.mark.parametrize("M,K_,N", [(4096, 320, 4096), (1020, 8200, 4100)])
+def test_split_product_outside_its_range(gpu, M, K_, N, special):
+    """Values that the parts cannot represent take the fp32 kernel: the same
+    infinities and NaN as the fp32 product, and full relative precision of
+    large, tiny and mixed magnitudes; zeros stay in range."""
+    r = rng(seed_of("split-range", M, special))
+    a = r.standard_normal((M, K_), dtype=np.float32)
+    b = r.standard_normal((K_, N), dtype=np.float32)
+    if special in ("inf", "nan"):
+        a[17, 5] = np.inf if special == "inf" else np.nan
+    elif special == "large":
+        a *= np.float32(1e30)
+    elif special == "tiny":
+        a *= np.float32(1e-30)
+    elif special == "tiny row":
+        a[17] *= np.float32(1e-30)
+    elif special == "both small":
+        a *= np.float32(1e-15)
+        b *= np.float32(1e-15)
+    else:
+        a[::3] = 0.0
+        b[:, ::2] = -0.0
+    got = host(nt.Tensor._new_contiguous(K.matmul(dev(a), dev(b), (M, N)), (M, N)))
+    if special in ("inf", "nan"):
+        with np.errstate(invalid="ignore"):
+            row = a[17].astype(np.float64) @ b
+        assert (np.isnan(got[17]) == np.isnan(row)).all()
+        assert (np.isinf(got[17]) == np.isinf(row)).all()
+        a, got = np.delete(a, 17, 0), np.delete(got, 17, 0)
+    want = a.astype(np.float64) @ b
+    scale = np.abs(a).astype(np.float64) @ np.abs(b)
+    assert (np.abs(got - want) <= K_ * 2.0**-24 * scale).all()
