@@ -543,6 +543,8 @@ def reshape_view(x: Tensor, dims: TensorShape) -> Tensor:
     contiguous; x itself if nothing changes."""
     if dims == x._shape:
         return x
+    if math.prod(dims) != x.numel:
+        raise ValueError(f"Can't reshape {x._shape} into {dims}.")
     x = x._to_contiguous()
     return Tensor._new_view(x._storage, dims, None, x._offset)
 

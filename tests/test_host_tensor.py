@@ -33,3 +33,15 @@ def test_from_numpy_with_dtype_override():
     t = nt.Tensor(a, dtype=nt.float32)
     assert t.dtype == nt.float32 and t.shape == (2, 3)
     assert t.cpu().tolist() == [[0.0, 1.0, 2.0], [3.0, 4.0, 5.0]]
+
+
+def test_reshape_view_refuses_another_size():
+    """The ops' reshape of a gradient, like Tensor.reshape: not a prefix of a
+    larger one."""
+    from nanotorch_amd.core import reshape_view
+
+    x = nt.Tensor(np.arange(12, dtype=np.float32))
+    assert reshape_view(x, (3, 4)).cpu().tolist() == np.arange(12.0).reshape(3, 4).tolist()
+    for dims in ((2, 4), (5,), (), (0,), (13,)):
+        with pytest.raises(ValueError):
+            reshape_view(x, dims)
