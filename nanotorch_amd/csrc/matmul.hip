@@ -618,6 +618,8 @@ __global__ __launch_bounds__(WD_THREADS, 1) void mm_f32_mfma_wide_kernel(
   const int lane = t & 63, wave = t >> 6;
   const int wm = wave >> 2, wn = wave & 3;
   const int h = lane >> 5, li = lane & 31;
+  if (g.flags && split_ok(g.flags) != g.run_if)
+    return;
   const TileCoord tc = mm_tile_coord<WD_BM, WD_BN>(g);
 
   floatx16 acc[4][2];
@@ -692,8 +694,10 @@ __global__ __launch_bounds__(WD_THREADS, 1) void mm_f32_mfma_wide_kernel(
 // added as for the other tiles.  What six exact products cannot do as the
 // fp32 kernel does -- infinities and NaN (0 x inf among the parts), parts or
 // products outside the normal range -- the pack kernel reports in a flag
-// word per operand: then mm_split_kernel returns at once and the fp32 tile
-// kernel, queued behind it, does the work; otherwise that one returns at once.
+// word per operand: then mm_split_kernel returns at once and the fp32
+// kernel queued behind it does the work; otherwise that one returns at once.
+// (Out of range, 8192x4096x4096 takes 2059 us, 1974 without the packing; 4000^3
+// 1116 / 1071; 1024x8192x4096 685 / 581, whose K is not split then.)
 constexpr int SP_B = 256, SP_K = 16;             // rows of a block, k of a step
 constexpr int SP_PLANE = SP_B * SP_K;            // bf16 values
 constexpr int SP_STEP = 3 * SP_PLANE * 2;        // bytes of a block's k step
@@ -909,8 +913,8 @@ __global__ __launch_bounds__(512, 1) void mm_split_kernel(
       for (int r = 0; r < 16; ++r) {
         const int64_t row =
             tc.m0 + wm * 128 + i * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
-        if (row < g.M)
-          mm_put(g, tc, row, col, acc[i][j][r]);
+        if (row < g.M) // + 0: a sum of zeros is +0, as in the fp32 kernels
+          mm_put(g, tc, row, col, acc[i][j][r] + 0.f);
       }
     }
 }
@@ -1309,7 +1313,8 @@ template <int LA, int LB> bool launch_wide(const MMArgs &a) {
   const int64_t tiles = a.M / WD_BM * (a.N / WD_BN) * a.nbatch;
   const int64_t cus = device_cu_count();
   int S = 1;
-  while (tiles * S < cus && a.nbatch == 1 && S < 8 && a.K % (64 * 2 * S) == 0 &&
+  // (unsplit as the fallback of a split product, as in launch_stages)
+  while (!a.flags && tiles * S < cus && a.nbatch == 1 && S < 8 && a.K % (64 * 2 * S) == 0 &&
          a.K / (2 * S) >= 1024)
     S *= 2;
   if (tiles * S < cus)
@@ -1431,6 +1436,12 @@ void launch_f32(const MMArgs &a, bool al) {
         b_mn ? launch_stages<ST_K4, ST_MN4>(g) : launch_stages<ST_K4, ST_K4>(g);
     }
   };
+  auto large = [&](const MMArgs &g) {
+    return wide && (a_mn ? (b_mn ? launch_wide<LAY_MN, LAY_MN>(g)
+                                 : launch_wide<LAY_MN, LAY_K>(g))
+                         : (b_mn ? launch_wide<LAY_K, LAY_MN>(g)
+                                 : launch_wide<LAY_K, LAY_K>(g)));
+  };
   if (!far && a.nbatch == 1) {
     // large tiles at 131 TFLOP/s, or the tile kernel's estimate (4-byte loads
     // at 0.8 of its rate)
@@ -1438,14 +1449,14 @@ void launch_f32(const MMArgs &a, bool al) {
     if (flops_us > 20) {
       const double est = choose_tile(a.M, a.N, a.K, 1).us;
       if (launch_split(a, wide ? std::max(flops_us, est) : 1.25 * std::max(flops_us, est),
-                       ak, bk, tiles))
+                       ak, bk, [&](const MMArgs &g) {
+                         if (!large(g))
+                           tiles(g);
+                       }))
         return;
     }
   }
-  if (wide && (a_mn ? (b_mn ? launch_wide<LAY_MN, LAY_MN>(a)
-                            : launch_wide<LAY_MN, LAY_K>(a))
-                    : (b_mn ? launch_wide<LAY_K, LAY_MN>(a)
-                            : launch_wide<LAY_K, LAY_K>(a))))
+  if (large(a))
     return;
   if (far) {
     MMArgs w = a;

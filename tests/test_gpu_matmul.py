@@ -470,3 +470,13 @@ def test_split_product_outside_its_range(gpu, M, K_, N, special):
     want = a.astype(np.float64) @ b
     scale = np.abs(a).astype(np.float64) @ np.abs(b)
     assert (np.abs(got - want) <= K_ * 2.0**-24 * scale).all()
+
+
+@pytest.mark.parametrize("K_", [320, 400])  # the last k step as it is, and packed negated
+def test_split_product_zero_sums_are_positive(gpu, K_):
+    """Sums of zeros are +0, as every float32 sum that starts at +0."""
+    a = np.zeros((4096, K_), np.float32)
+    a[::2] = -0.0
+    b = rng(seed_of("split-zero", K_)).standard_normal((K_, 4096), dtype=np.float32)
+    got = host(nt.Tensor._new_contiguous(K.matmul(dev(a), dev(b), (4096, 4096)), (4096, 4096)))
+    assert not got.any() and not np.signbit(got).any()
