@@ -1069,19 +1069,33 @@ def _mm_calls():
 
 def _mm_dispatches(rows):
     """Assigns matmul dispatches (dicts with Kernel_Name, in dispatch order)
-    to bench_matmul's calls: each call is one product kernel, followed by
-    the split-K sum kernel when K is split.  Yields (call, row, is_sum)."""
+    to bench_matmul's calls: a call is one product kernel, followed by the
+    split-K sum kernel when K is split; on bf16 planes it starts with the flag
+    and pack kernels and ends with the fp32 kernel that has nothing to do.
+    Yields (call, row, is_beside): beside the product kernel."""
     calls = _mm_calls()
     ci = -1
+    planes = ""  # the part of a call on bf16 planes that has been seen
     for r in rows:
         name = r["Kernel_Name"]
         if "mm_" not in name:
             continue
-        is_sum = "splitk_sum" in name
-        if not is_sum:
+        beside = True
+        if "mm_split_flags" in name:
             ci += 1
+            planes = "pack"
+        elif "mm_split_kernel" in name:
+            planes = "product"
+            beside = False
+        elif "mm_split_pack" in name or "splitk_sum" in name:
+            pass
+        elif planes == "product":
+            planes = ""
+        else:
+            ci += 1
+            beside = False
         if 0 <= ci < len(calls):
-            yield calls[ci], r, is_sum
+            yield calls[ci], r, beside
 
 
 SWEEP_TIMER_SWEEPS = 2  # bench_elementwise's per-kernel pass under PROFILE_CMDS["sweep"] (--steps 5)
@@ -1177,18 +1191,18 @@ def _summarize_next_trace(path: str, out_md: str) -> None:
 
 def _summarize_mm_trace(path: str, out_md: str) -> None:
     """Config-4 kernel times per product and shape from the kernel trace
-    (one row per (shape, A layout, product): the product kernel and, with
-    split K, the sum kernel), timed rounds only, as bench_matmul reports."""
+    (one row per (shape, A layout, product): the product kernel and the ones
+    beside it, i.e. the split-K sum and the packing of planes), timed rounds only, as bench_matmul reports."""
     import csv
     rows = sorted(csv.DictReader(open(os.path.join(path, "run_kernel_trace.csv"))),
                   key=lambda r: int(r["Dispatch_Id"]))
     acc: dict = {}
-    for (M, Kd, N, lay, prod, warm), r, is_sum in _mm_dispatches(rows):
+    for (M, Kd, N, lay, prod, warm), r, beside in _mm_dispatches(rows):
         if warm:
             continue
         e = acc.setdefault((M, Kd, N, lay, prod), {"main": [], "sum": [], "name": "", "grid": ""})
         us = (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3
-        if is_sum:
+        if beside:
             e["sum"].append(us)
         else:
             e["main"].append(us)
@@ -1200,14 +1214,15 @@ def _summarize_mm_trace(path: str, out_md: str) -> None:
         o.write("Summarised with `python bench.py --summarize mm gpurun_out/prof_mm` from the "
                 "kernel trace: each dispatch is matched to bench_matmul's call sequence (per shape, "
                 "per A layout, rounds of fwd, dA = dG.B^T, dB = A^T.dG; the first round untimed), "
-                "so the two config-4 shapes get rows of their own.  `sum us` is the split-K sum "
-                "kernel where K is split; TFLOP/s = 2MNK / (product + sum).  Grid in work-items "
-                "(x by split-K slices).\n\n")
-        o.write("| shape MxKxN | A | product | kernel | grid | n | product us | sum us | TFLOP/s | frac of 157.3 |\n"
+                "so the two config-4 shapes get rows of their own.  `beside us` is the call's other "
+                "kernels: the split-K sum where K is split, and for a product on bf16 planes the "
+                "packing and the fp32 kernel that returns at once; TFLOP/s = 2MNK / (product + "
+                "beside).  Grid in work-items.\n\n")
+        o.write("| shape MxKxN | A | product | kernel | grid | n | product us | beside us | TFLOP/s | frac of 157.3 |\n"
                 "|---|---|---|---|---|---|---|---|---|---|\n")
         for (M, Kd, N, lay, prod), e in acc.items():
             mu = sum(e["main"]) / len(e["main"])
-            su = sum(e["sum"]) / len(e["sum"]) if e["sum"] else 0.0
+            su = sum(e["sum"]) / len(e["main"])
             m_, k_, n_ = {"fwd": (M, Kd, N), "dA": (M, N, Kd), "dB": (Kd, M, N)}[prod]
             tf = 2.0 * m_ * n_ * k_ / ((mu + su) * 1e-6) / 1e12
             o.write(f"| {M}x{Kd}x{N} | {lay} | {prod} | `{e['name'][:60]}` | {e['grid']} | {len(e['main'])} | "
@@ -1228,8 +1243,8 @@ def _summarize_mm_pmc(path: str, out_md: str) -> None:
         d[r["Counter_Name"]] = float(r["Counter_Value"])
     rows = [disp[k] for k in sorted(disp)]
     per: dict = {}
-    for (M, Kd, N, lay, prod, warm), d, is_sum in _mm_dispatches(rows):
-        if warm or is_sum:
+    for (M, Kd, N, lay, prod, warm), d, beside in _mm_dispatches(rows):
+        if warm or beside:
             continue
         per.setdefault((M, Kd, N, lay, prod), []).append(d)
     with open(out_md, "w") as o:
@@ -1237,10 +1252,11 @@ def _summarize_mm_pmc(path: str, out_md: str) -> None:
         o.write(f"Command (repo root on the GPU box):\n\n```\n{PROFILE_CMDS['mm_pmc']}\n```\n\n")
         o.write("Summarised with `python bench.py --summarize mm_pmc gpurun_out/prof_mm_pmc`; "
                 "each dispatch is matched to bench_matmul's call sequence, timed rounds only, "
-                "the product kernel alone (a split-K sum kernel has no MFMA). "
+                "the product kernel alone (the kernels beside it have no MFMA). "
                 "Utilisation = SQ_VALU_MFMA_BUSY_CYCLES (summed over the 1024 SIMDs) / "
-                "(1024 x kernel duration x 2.4 GHz); each v_mfma_f32_32x32x2_f32 keeps the "
-                "pipe busy 64 cycles, so this equals achieved / peak FLOP rate at 2.4 GHz. "
+                "(1024 x kernel duration x 2.4 GHz): the share of the peak rate of the unit "
+                "that the kernel runs on, at 2.4 GHz (mm_split_kernel: bf16, six products per "
+                "fp32 one; the others: fp32). "
                 "Durations are from this (counter-collecting) run.\n\n")
         o.write("| shape MxKxN | A | product | kernel | grid | n | avg us | MFMA instr | MFMA util | "
                 "LDS-wait / wave cycles | LDS bank conflicts |\n"
