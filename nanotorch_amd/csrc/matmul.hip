@@ -708,7 +708,7 @@ constexpr int SP_STEP = 3 * SP_PLANE * 2;        // bytes of a block's k step
 // the sign changes: down is then up, and the shifts cancel.  The signs follow
 // the parity of the run number's bits (+ - - + - + + -), which cancels the
 // growth of the sums, and of their roundings, along K as well.
-constexpr uint32_t SP_FLIP = 6; // a multiple of the k loop's 3
+constexpr uint32_t SP_FLIP = 3; // a multiple of the k loop's 3
 __device__ __forceinline__ bool split_negated(uint32_t step) {
   return __popc(step / SP_FLIP) & 1;
 }
@@ -863,8 +863,10 @@ __global__ __launch_bounds__(512, 1) void mm_split_kernel(
   // wait leaves the 6 loads of the step after next in flight.  Past the end
   // the last step is loaded again, to keep the count.  steps is a multiple
   // of 3: one exit, so that the accumulators stay where they are.
+  // lgkmcnt(0): this wave's reads of the stage that is loaded next are done
+  // (the MFMAs that wait for them may be scheduled past the barrier).
   auto landed = [] {
-    asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
