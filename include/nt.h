@@ -302,6 +302,13 @@ int nt_matmul(const nt_view *a, const nt_view *b, const nt_view *c,
 int nt_matmul_bias(const nt_view *a, const nt_view *b, const nt_view *bias,
                    const nt_view *c);
 
+/* nt_matmul_bias on the fp32 matrix cores at every size (nt_matmul and
+ * nt_matmul_bias run large single products on the bf16 ones, whose results
+ * differ in the last bits): a linear layer's forward, whose rounding decides
+ * which side of a following ReLU's corner a value falls on. */
+int nt_linear(const nt_view *x, const nt_view *w, const nt_view *bias,
+              const nt_view *y);
+
 /* --------------------------------------------------------------- indexing */
 
 /* Replaces `gather_from_axes` (src/cpp/ops/copy_ops.cu:93-160, host only in

@@ -326,6 +326,15 @@ def matmul_bias(x1, x2, bias, out_shape) -> Storage:
     return out
 
 
+def linear(x, w, bias, out_shape) -> Storage:
+    """matmul_bias on the fp32 kernels at every size: a layer's forward."""
+    require_device(x, w, bias)
+    out = Storage.allocate(_numel(out_shape), x.dtype, Device.Cuda)
+    _lib.call_packed("nt_linear", _packed(x), _packed(w), _packed(bias),
+                     _packed_flat(out, out_shape))
+    return out
+
+
 def matmul_into(x1, x2, target, accumulate: bool) -> None:
     require_device(x1, x2, target)
     v1, v2, vo = _packed(x1), _packed(x2), _packed(target)

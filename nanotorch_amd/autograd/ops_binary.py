@@ -245,9 +245,10 @@ class MatmulOp(Function):
 
 class LinearOp(Function):
     """x @ W + b for 2-D float32 device operands in one product whose
-    epilogue adds b (nt_matmul_bias): the reference's Linear forward, a
+    epilogue adds b (nt_linear): the reference's Linear forward, a
     MatmulOp then an AddOp (src/nanotorch/nn/module.py:73-75), with the same
-    two fp32 roundings (the product's, then the add's).  Its backward is
+    two fp32 roundings (the product's, then the add's; a large product of a
+    MatmulOp runs on another unit and differs in its last bits).  Its backward is
     those two ops' backward: dx = g . W^T and dW = x^T . g (MatmulOp,
     src/nanotorch/autograd/ops_binary.py:253-267, each one product reading
     the transposed operand in place), db = g summed over the rows (AddOp's
@@ -257,7 +258,7 @@ class LinearOp(Function):
         self.save_for_backward(x, W)
         self._b_shape = b.shape
         shape = (x.shape[0], W.shape[1])
-        return Tensor._new_contiguous(K.matmul_bias(x, W, b, shape), shape)
+        return Tensor._new_contiguous(K.linear(x, W, b, shape), shape)
 
     def backward(self, grad_out: Tensor) -> tuple[Tensor, ...]:
         x, W = self.saved_tensors

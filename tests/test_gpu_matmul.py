@@ -480,3 +480,17 @@ def test_split_product_zero_sums_are_positive(gpu, K_):
     b = rng(seed_of("split-zero", K_)).standard_normal((K_, 4096), dtype=np.float32)
     got = host(nt.Tensor._new_contiguous(K.matmul(dev(a), dev(b), (4096, 4096)), (4096, 4096)))
     assert not got.any() and not np.signbit(got).any()
+
+
+def test_layer_forward_keeps_the_fp32_rounding(gpu):
+    """A layer's forward at a size whose plain product takes the planes: bit
+    for bit the values of a run in which another row's infinity keeps that
+    product on the fp32 kernel."""
+    from nanotorch_amd import nn
+    r = rng(seed_of("layer-forward"))
+    lin = nn.Linear(1024, 4096)
+    lin._W = dev(r.standard_normal((1024, 4096), dtype=np.float32) / np.float32(32))
+    x = r.standard_normal((4096, 1024), dtype=np.float32)
+    clean = host(lin(dev(x)))
+    x[17, 5] = np.inf
+    assert_bitexact(np.delete(clean, 17, 0), np.delete(host(lin(dev(x))), 17, 0), "forward")
