@@ -678,15 +678,31 @@ __global__ __launch_bounds__(WD_THREADS, 1) void mm_f32_mfma_wide_kernel(
 // A float32 is the exact sum of three bfloat16 values (8 + 8 + 8 bits of
 // significand), and a product of bfloat16 values is exact in float32.  So
 // a . b = (a1 + a2 + a3) . (b1 + b2 + b3) can run on the bf16 MFMA, which does
-// 16 times the work of the fp32 one per cycle, accumulating in float32 as
-// before: six of the nine products, the three left out (a2 b3, a3 b2, a3 b3)
-// are below 2^-26 of a b, under the rounding of a float32 product.
-// Error against 64 bits (2-norm), fp32 MFMA -> this: normal operands 4096^3
-// 1.15e-6 -> 9.7e-7, 4096x1000x4096 5.7e-7 -> 4.8e-7, 4096x320x4096 3.2e-7 ->
-// 2.7e-7, 1024x8192x4096 8.1e-7 -> 6.9e-7; uniform [0, 1) 4096^3 8.4e-7 ->
-// 5.2e-7: 6 roundings of the sum per 16 k's where the fp32 MFMA has 8 and the
-// products' own.  Mean shift of the results: at most 7e-9 of their mean
-// magnitude (4e-9 before).
+// 16 times the work of the fp32 one per cycle (Henry, Tang and Heinecke,
+// "Leveraging the bfloat16 Artificial Intelligence Datatype for Higher-
+// Precision Computations", 2019): six of the nine products.  Of the three left
+// out a2 b3 and a3 b2 are at most 2^-25 of a b each (2^-29 of it together in
+// the median of normal operands, 2^-24 at most), half an ulp of a float32.
+//
+// Rounding: the bf16 MFMA rounds its sums down (towards -infinity), so no
+// running sum of K stays in it.  The leading products a1 b1 of 32 k's are
+// summed on the matrix cores (exactly, for a few terms of like size), and the
+// vector unit adds that to the running sum, to nearest: one rounding of the
+// sum per 32 k's, where the fp32 MFMA has 16.  Every other pair of steps the
+// leading products are formed negated and subtracted: what is rounded down is
+// then rounded up, and the results have no mean shift.  The five small
+// products, 2^-8 of the leading one, have accumulators of their own on the
+// matrix cores, which join the sum at the end: their roundings are 2^-8 of a
+// float32's.
+//
+// Error against 64 bits, fp32 MFMA -> this, 2-norm: normal operands 4000^3
+// 1.13e-6 -> 2.1e-7, 4096x300x4096 3.1e-7 -> 7.3e-8, 1024x8192x4096 8.1e-7 ->
+// 2.1e-7 (51 non-zeros to a row of 8192: 8.0e-8 -> 5.1e-8); positive operands
+// 8192x4096x4096 8.8e-7 -> 1.6e-7.  Mean shift of the results within 5e-10 of
+// their mean magnitude (1e-9); of one column's mean 2e-7 (1.1e-6).  Sums of a
+// single term, in 2^-24 of it: exact for a one-hot operand, largest error
+// 1.0 -> 1.8 and rms 0.425 -> 0.436 for a diagonal one (the products left
+// out); of two terms, rms 0.436 -> 0.368.
 //
 // Three kernels: mm_split_pack_kernel writes both operands as packed bf16
 // planes, in the order in which the product's LDS stages hold them, zeros
@@ -701,18 +717,8 @@ __global__ __launch_bounds__(WD_THREADS, 1) void mm_f32_mfma_wide_kernel(
 constexpr int SP_B = 256, SP_K = 16;             // rows of a block, k of a step
 constexpr int SP_PLANE = SP_B * SP_K;            // bf16 values
 constexpr int SP_STEP = 3 * SP_PLANE * 2;        // bytes of a block's k step
-// The bf16 MFMA rounds its sums down (towards -infinity): left alone, results
-// are 2.6e-7 of their mean magnitude too low, which does not average out in
-// what sums them next (a loss, a bias gradient).  So A's values are packed
-// negated in half of the runs of SP_FLIP steps, and the sums are negated where
-// the sign changes: down is then up, and the shifts cancel.  The signs follow
-// the parity of the run number's bits (+ - - + - + + -), which cancels the
-// growth of the sums, and of their roundings, along K as well.
-constexpr uint32_t SP_FLIP = 3; // a multiple of the k loop's 3
-__device__ __forceinline__ bool split_negated(uint32_t step) {
-  return __popc(step / SP_FLIP) & 1;
-}
-
+constexpr int SP_BN = 128;                       // columns of a tile
+constexpr int SP_STAGE = SP_STEP + SP_STEP / 2;  // LDS of one step of a tile
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 __global__ void mm_split_flags_kernel(uint32_t *flags) {
@@ -762,16 +768,14 @@ __global__ __launch_bounds__(256) void mm_split_pack_kernel(
   }
   bf16x8 p1, p2, p3;
   uint32_t f = 0;
-  const bool neg = !second && split_negated(step);
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const uint32_t ex = (__float_as_uint(v[e]) >> 23) & 255; // 127: 1.x
     const bool zero = v[e] == 0.f;
     f |= ex >= 127 + 50 || (!zero && ex < 127 - 60) ? SP_BAD : 0;
     f |= !zero && ex < 127 - 40 ? SP_SMALL : 0;
-    const float x = neg ? -v[e] : v[e];
-    p1[e] = __bf16(x);
-    const float r = x - float(p1[e]);
+    p1[e] = __bf16(v[e]);
+    const float r = v[e] - float(p1[e]);
     p2[e] = __bf16(r);
     p3[e] = __bf16(r - float(p2[e]));
   }
@@ -784,128 +788,155 @@ __global__ __launch_bounds__(256) void mm_split_pack_kernel(
     atomicOr(flags + second, f);
 }
 
-// 256x256 tiles, 8 waves in a 2x4 grid (two per SIMD) of 128x64: 4x2 blocks
-// of 32x32, 48 MFMAs of 32x32x16 per k step against 18 fragment reads, so
-// the matrix pipe, not LDS, is the bound.  Stages are copies of the packed
+// 256x128 tiles, 8 waves in a 4x2 grid (two per SIMD) of 64x64: 2x2 blocks of
+// 32x32 in two sets of accumulators (128 registers) and the leading products
+// of two steps (64 more), 24 MFMAs of 32x32x16 per k step against 12 fragment
+// reads (half of the LDS rate), so the matrix pipe and the chip's power (the
+// clock falls below 2 GHz) are the bound.  Stages are copies of the packed
 // operands (every load 1 KB of consecutive memory, conflict-free reads).
-// Three stages keep the matrix pipe busy 84% of cycles (two: 75%), at which
-// the chip's power, not the kernel, sets the rate: the clock falls to 1.8 GHz.
-// 8192x4096x4096 with packing: 1930 us on the fp32 MFMA, 1200 here (229
-// TFLOP/s; 1232 with two stages); 4000^3 1062 -> 611 us, 8192x4096x1000 in two
-// slices of K 553 -> 368, 4096x300x4096 106 -> 71.
+// With packing, in us, fp32 MFMA -> this: 8192x4096x4096 1980 -> 1393,
+// 4000^3 1075 -> 738, 1024x8192x4096 510 -> 420, 8192x4096x1000 520 -> 398,
+// 4096x300x4096 109 -> 81.  (One running sum of all six products in 256x256
+// tiles, every sum rounded down: 4000^3 682 us, with five times the error; the
+// leading products of each step added apart: 759.)
 __global__ __launch_bounds__(512, 1) void mm_split_kernel(
     MMArgs g, const char *pa, const char *pb, uint32_t ksteps, uint32_t kper,
     const uint32_t *flags) {
   if (!split_ok(flags))
     return;
-  __shared__ __align__(16) char sA0[SP_STEP], sB0[SP_STEP];
-  __shared__ __align__(16) char sA1[SP_STEP], sB1[SP_STEP];
-  __shared__ __align__(16) char sA2[SP_STEP], sB2[SP_STEP];
+  __shared__ __align__(16) char st0[SP_STAGE], st1[SP_STAGE], st2[SP_STAGE], st3[SP_STAGE];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wave >> 2, wn = wave & 3;
-  const TileCoord tc = mm_tile_coord<SP_B, SP_B>(g);
-  floatx16 acc[4][2];
+  const int wm = wave >> 1, wn = wave & 1;
+  const TileCoord tc = mm_tile_coord<SP_B, SP_BN>(g);
+  // the sum of the leading products, that of the five small ones, and the
+  // leading products of the present pair of steps
+  floatx16 acc[2][2], low[2][2], top[2][2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r)
-        acc[i][j][r] = 0.f;
+        acc[i][j][r] = low[i][j][r] = 0.f;
   const uint32_t s0 = tc.slice * kper;
   const uint32_t steps = ksteps - s0 < kper ? ksteps - s0 : kper;
   const char *a0 = pa + (tc.m0 / SP_B * ksteps + s0) * SP_STEP;
   const char *b0 = pb + (tc.n0 / SP_B * ksteps + s0) * SP_STEP;
-  auto issue = [&](char *sa, char *sb, uint32_t s) {
-    // a wave copies 3 KB of each operand's 24
-    auto copy = [&](char *stage, const char *src) {
-      const uint64_t ub = reinterpret_cast<uint64_t>(src + int64_t(s) * SP_STEP);
+  // A stage is A's step (24 KB) and B's half of one (3 planes of 4 KB): 36
+  // pieces of 1 KB, piece 8 j + wave by this wave (the last 4 twice: every
+  // wave then has 5 loads in flight per stage).
+  const uint32_t bhalf = uint32_t(tc.n0 / SP_BN % 2) * SP_PLANE;
+  auto issue = [&](char *stage, uint32_t s) {
+    auto rsrc = [](const char *src) {
+      const uint64_t ub = reinterpret_cast<uint64_t>(src);
       const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(ub));
       const uint32_t hi = __builtin_amdgcn_readfirstlane(uint32_t(ub >> 32));
-      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      return __builtin_amdgcn_make_buffer_rsrc(
           reinterpret_cast<void *>((uint64_t(hi) << 32) | lo), 0, SP_STEP, BUF_WORD3);
-#pragma unroll
-      for (int j = 0; j < 3; ++j)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rs,
-            (__attribute__((address_space(3))) void *)(stage + (wave * 3 + j) * 1024),
-            16, (wave * 3 + j) * 1024 + lane * 16, 0, 0, 0);
     };
-    copy(sa, a0);
-    copy(sb, b0);
+    const __amdgpu_buffer_rsrc_t ra = rsrc(a0 + int64_t(s) * SP_STEP);
+    const __amdgpu_buffer_rsrc_t rb = rsrc(b0 + int64_t(s) * SP_STEP);
+#pragma unroll
+    for (int j = 0; j < 5; ++j) {
+      if (j < 3) {
+        const int piece = 8 * j + wave;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            ra, (__attribute__((address_space(3))) void *)(stage + piece * 1024), 16,
+            piece * 1024 + lane * 16, 0, 0, 0);
+      } else {
+        const int q = j == 3 ? wave : 8 + wave % 4; // piece of B
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            rb, (__attribute__((address_space(3))) void *)(stage + SP_STEP + q * 1024),
+            16, (q / 4) * (2 * SP_PLANE) + bhalf + (q % 4) * 1024 + lane * 16, 0, 0, 0);
+      }
+    }
   };
-  auto compute = [&](const char *sa, const char *sb) {
-    bf16x8 a[4][3], b[2][3];
+  // NEG: the pair's leading products are formed negated; LAST: its second step.
+  auto compute = [&]<bool NEG, bool LAST>(const char *st) {
+    bf16x8 a[2][3], b[2][3], b1[2];
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        a[i][p] = *reinterpret_cast<const bf16x8 *>(sa + p * 2 * SP_PLANE +
-                                                    (wm * 4 + i) * 1024 + lane * 16);
+      for (int i = 0; i < 2; ++i)
+        a[i][p] = *reinterpret_cast<const bf16x8 *>(st + p * 2 * SP_PLANE +
+                                                    (wm * 2 + i) * 1024 + lane * 16);
 #pragma unroll
       for (int j = 0; j < 2; ++j)
-        b[j][p] = *reinterpret_cast<const bf16x8 *>(sb + p * 2 * SP_PLANE +
+        b[j][p] = *reinterpret_cast<const bf16x8 *>(st + SP_STEP + p * SP_PLANE +
                                                     (wn * 2 + j) * 1024 + lane * 16);
     }
-    // small products first
-    constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
-    for (int q = 0; q < 6; ++q)
+    for (int j = 0; j < 2; ++j) {
+      b1[j] = b[j][0];
+      if constexpr (NEG) {
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+        b1[j] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, b1[j]) ^ 0x80008000u);
+      }
+    }
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        top[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            a[i][0], b1[j], LAST ? top[i][j] : floatx16{}, 0, 0, 0);
+    constexpr int PA[5] = {2, 0, 1, 1, 0}, PB[5] = {0, 2, 1, 0, 1};
+#pragma unroll
+    for (int q = 0; q < 5; ++q)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              a[i][PA[q]], b[j][PB[q]], acc[i][j], 0, 0, 0);
+          low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][PA[q]], b[j][PB[q]],
+                                                              low[i][j], 0, 0, 0);
+    if constexpr (LAST)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            acc[i][j][r] = NEG ? acc[i][j][r] - top[i][j][r] : acc[i][j][r] + top[i][j][r];
   };
-  // Three stages: a step's loads have two steps of MFMAs to land in, so the
-  // wait leaves the 6 loads of the step after next in flight.  Past the end
-  // the last step is loaded again, to keep the count.  steps is a multiple
-  // of 3: one exit, so that the accumulators stay where they are.
+  // Four stages: a step's loads have three steps of MFMAs to land in, so the
+  // wait leaves the 10 loads of the two steps after next in flight.  Past the
+  // end the last step is loaded again, to keep the count.  steps is a
+  // multiple of 4: one exit, so that the accumulators stay where they are.
   // lgkmcnt(0): this wave's reads of the stage that is loaded next are done
   // (the MFMAs that wait for them may be scheduled past the barrier).
   auto landed = [] {
-    asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(10) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
   auto at = [&](uint32_t s) { return s < steps ? s : steps - 1; };
-  issue(sA0, sB0, 0);
-  issue(sA1, sB1, 1);
+  issue(st0, 0);
+  issue(st1, 1);
+  issue(st2, 2);
   landed();
-  auto negate = [&] {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          acc[i][j][r] = -acc[i][j][r];
-  };
-  for (uint32_t s = 0; s < steps; s += 3) {
-    if (s > 0 && split_negated(s0 + s) != split_negated(s0 + s - 1))
-      negate();
-    issue(sA2, sB2, s + 2);
+  for (uint32_t s = 0; s < steps; s += 4) {
+    issue(st3, s + 3);
     pin_issued_loads();
-    compute(sA0, sB0);
+    compute.template operator()<false, false>(st0);
     landed();
-    issue(sA0, sB0, at(s + 3));
+    issue(st0, at(s + 4));
     pin_issued_loads();
-    compute(sA1, sB1);
+    compute.template operator()<false, true>(st1);
     landed();
-    issue(sA1, sB1, at(s + 4));
+    issue(st1, at(s + 5));
     pin_issued_loads();
-    compute(sA2, sB2);
+    compute.template operator()<true, false>(st2);
+    landed();
+    issue(st2, at(s + 6));
+    pin_issued_loads();
+    compute.template operator()<true, true>(st3);
     landed();
   }
-  if (split_negated(s0 + steps - 1))
-    negate();
   // no load may still write the LDS of a workgroup that has ended
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   const int h = lane >> 5, li = lane & 31;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int64_t col = tc.n0 + wn * 64 + j * 32 + li;
@@ -914,9 +945,9 @@ __global__ __launch_bounds__(512, 1) void mm_split_kernel(
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int64_t row =
-            tc.m0 + wm * 128 + i * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
+            tc.m0 + wm * 64 + i * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
         if (row < g.M) // + 0: a sum of zeros is +0, as in the fp32 kernels
-          mm_put(g, tc, row, col, acc[i][j][r] + 0.f);
+          mm_put(g, tc, row, col, acc[i][j][r] + low[i][j][r] + 0.f);
       }
     }
 }
@@ -1332,28 +1363,31 @@ template <int LA, int LB> bool launch_wide(const MMArgs &a) {
 }
 
 // The product through packed bf16 planes (mm_split_kernel), where that is
-// estimated to take less than 0.92 of the fp32 time f32_us; false: not taken.
-// A k step of a tile takes 1.5 us with few CUs at work and 2.1 with all (the
-// clock falls with the power), packing 10 bytes per value at 5 TB/s and the
-// three small launches 12 us; measured against the estimate: 4000^3 611 us /
-// 616, 8192x4096x1000 368 / 390, 1024x8192x4096 388 / 396, 4096x300x4096
-// 71 / 69.  ak, bk: the operand has 16-byte aligned rows along k.
+// estimated to take no longer than the fp32 kernels' f32_us (an estimate too,
+// of 0.8 to 1 of what they measured); false: not taken.  A k step of a tile
+// takes 0.8 us with few CUs at work and 1.12 with all (the clock falls with
+// the power), packing 10 bytes per value at 5 TB/s and the three small
+// launches 12 us; measured / estimated / fp32 measured, in us: 4000^3 665 /
+// 660 / 1050, 8192x4096x1000 388 / 383 / 572, 1024x8192x4096 410 / 404 / 556,
+// 2912x2804x6472 625 / 646 / 900, 4093x301x4090 80 / 80 / 118.  ak, bk: the
+// operand has 16-byte aligned rows along k.
 template <class FB>
 bool launch_split(const MMArgs &a, double f32_us, bool ak, bool bk, FB fallback) {
   if (f32_us < 40 || a.K >= (int64_t(1) << 27))
     return false;
   const int64_t tm = ceil_div(a.M, SP_B), tn = ceil_div(a.N, SP_B);
-  const int64_t ksteps = ceil_div(a.K, 3 * SP_K) * 3; // in threes, see the kernel
+  const int64_t ksteps = ceil_div(a.K, 4 * SP_K) * 4; // in fours, see the kernel
+  const int64_t tiles = tm * ceil_div(a.N, SP_BN);
   const int64_t cus = device_cu_count();
   const double outs = double(a.M) * double(a.N);
   double best_t = std::numeric_limits<double>::infinity();
   int S = 1;
   for (int s : {1, 2, 3, 4, 6, 8}) {
-    const int64_t per = ceil_div(ksteps, 3 * s) * 3;
+    const int64_t per = ceil_div(ksteps, 4 * s) * 4;
     if (ceil_div(ksteps, per) != s)
       continue;
-    const double busy = std::min(1.0, double(tm * tn * s) / double(cus));
-    double t = double(ceil_div(tm * tn * s, cus)) * (double(per) * (1.5 + 0.6 * busy) + 8);
+    const double busy = std::min(1.0, double(tiles * s) / double(cus));
+    double t = double(ceil_div(tiles * s, cus)) * (double(per) * (0.8 + 0.32 * busy) + 9);
     if (s > 1)
       t += 4 + (s + 1) * outs * 4 / 6e6;
     if (t < best_t) {
@@ -1362,11 +1396,11 @@ bool launch_split(const MMArgs &a, double f32_us, bool ak, bool bk, FB fallback)
     }
   }
   const double pack = 12 + double(tm + tn) * SP_B * double(a.K) * 10 / 5e6;
-  if (best_t + pack > 0.92 * f32_us)
+  if (best_t + pack > f32_us)
     return false;
   const size_t abytes = size_t(tm * ksteps) * SP_STEP, bbytes = size_t(tn * ksteps) * SP_STEP;
   const size_t pbytes = S > 1 ? size_t(S) * size_t(outs) * sizeof(float) : 0;
-  if (outs >= 4294967296. || tm * tn * S >= (int64_t(1) << 31) ||
+  if (outs >= 4294967296. || tiles * S >= (int64_t(1) << 31) ||
       (tm + tn) * 8 * ceil_div(ksteps, 4) >= (int64_t(1) << 31))
     return false;
   void *scratch = nullptr;
@@ -1393,10 +1427,10 @@ bool launch_split(const MMArgs &a, double f32_us, bool ak, bool bk, FB fallback)
   NT_LAUNCH_CHECK();
   MMArgs w = a;
   w.tiles_m = tm;
-  w.tiles_n = tn;
+  w.tiles_n = ceil_div(a.N, SP_BN);
   w.part = S > 1 ? reinterpret_cast<float *>(pb + bbytes) : nullptr;
-  mm_split_kernel<<<unsigned(tm * tn * S), 512, 0, stream()>>>(
-      w, pa, pb, uint32_t(ksteps), uint32_t(ceil_div(ksteps, 3 * S) * 3), flags);
+  mm_split_kernel<<<unsigned(tiles * S), 512, 0, stream()>>>(
+      w, pa, pb, uint32_t(ksteps), uint32_t(ceil_div(ksteps, 4 * S) * 4), flags);
   NT_LAUNCH_CHECK();
   w.flags = flags;
   if (S > 1) {

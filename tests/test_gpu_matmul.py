@@ -494,3 +494,60 @@ def test_layer_forward_keeps_the_fp32_rounding(gpu):
     clean = host(lin(dev(x)))
     x[17, 5] = np.inf
     assert_bitexact(np.delete(clean, 17, 0), np.delete(host(lin(dev(x))), 17, 0), "forward")
+
+
+def _sparse_operand(kind, n, r):
+    a = np.zeros((n, n), np.float32)
+    i = np.arange(n)
+    if kind == "one-hot":
+        a[i, r.permutation(n)] = 1
+    else:
+        a[i, i] = r.standard_normal(n, dtype=np.float32)
+    if kind == "two terms":
+        a[i, (7 * i + 3) % n] = r.standard_normal(n, dtype=np.float32)
+    return a
+
+
+@pytest.mark.parametrize("kind,most,rms", [("one-hot", 0, 0), ("diagonal", 2, 0.45),
+                                           ("two terms", 3, 0.45)])
+def test_split_product_of_few_terms(gpu, kind, most, rms):
+    """Plane products whose sums have one or two terms, where the running
+    sum's rounding does not hide a product's own.  In 2^-24 (|A|.|B|): each
+    rounding of the sum is at most 1, the products of parts left out 1 in
+    all, the five small products' roundings 1/16; a one-hot operand's parts
+    are exact.  rms of one rounding to nearest
+    0.425 (a value uniform in an ulp, its size log-uniform); the fp32 kernel
+    has 0.425 and 0.436 for one and two terms."""
+    n = 4096
+    r = rng(seed_of("split-few", kind))
+    a = _sparse_operand(kind, n, r)
+    b = r.standard_normal((n, n), dtype=np.float32)
+    got = _mm(dev(a), dev(b))
+    want = a.astype(np.float64) @ b
+    err = np.abs(got - want) * 2.0**24
+    scale = np.abs(a).astype(np.float64) @ np.abs(b)
+    assert (err <= (most + 1 / 16 if most else 0) * scale).all()
+    q = err[scale > 0] / scale[scale > 0]
+    assert np.sqrt(np.mean(q * q)) <= rms
+
+
+@pytest.mark.parametrize("K_", [320, 4096])
+@pytest.mark.parametrize("dist", ["normal", "positive"])
+def test_split_product_has_no_mean_shift(gpu, dist, K_):
+    """The matrix cores round the planes' sums down; over 16 million results
+    what is left of that is below 2^-29 of their mean size (left alone it was
+    2.6e-7, over 2^-22), and a column's mean is no
+    further from 64 bits than its 4096 roundings to nearest allow."""
+    r = rng(seed_of("split-shift", dist, K_))
+    a = r.standard_normal((4096, K_), dtype=np.float32)
+    b = r.standard_normal((K_, 4096), dtype=np.float32) / np.float32(np.sqrt(K_))
+    if dist == "positive":
+        a, b = np.abs(a), np.abs(b)
+    got = _mm(dev(a), dev(b))
+    want = a.astype(np.float64) @ b
+    err = got - want
+    assert abs(err.mean()) <= 2.0**-29 * np.abs(want).mean()
+    # one rounding per 32 k's and two at the end, of sums no larger than the
+    # rows' largest; independent ones: 4.5 of their standard deviations
+    per = np.sqrt(K_ / 32 + 2) * 2.0**-24 * np.abs(want).max() / np.sqrt(3 * 4096)
+    assert np.abs(err.mean(0)).max() <= 4.5 * per
