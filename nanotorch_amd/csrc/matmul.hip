@@ -1308,9 +1308,7 @@ void launch_tile(const MMArgs &a, const TileChoice &c) {
 }
 
 template <int SA, int SB> void launch_stages(const MMArgs &a) {
-  // (as the fallback of a split product: rarely run, so unsplit)
-  const TileChoice c = a.flags ? TileChoice{128, 128, 1, a.K, 0}
-                               : choose_tile(a.M, a.N, a.K, a.nbatch);
+  const TileChoice c = choose_tile(a.M, a.N, a.K, a.nbatch);
   if (c.bm == 64)
     launch_tile<SA, SB, 64, 64>(a, c);
   else if (c.bm == 32)
@@ -1346,8 +1344,7 @@ template <int LA, int LB> bool launch_wide(const MMArgs &a) {
   const int64_t tiles = a.M / WD_BM * (a.N / WD_BN) * a.nbatch;
   const int64_t cus = device_cu_count();
   int S = 1;
-  // (unsplit as the fallback of a split product, as in launch_stages)
-  while (!a.flags && tiles * S < cus && a.nbatch == 1 && S < 8 && a.K % (64 * 2 * S) == 0 &&
+  while (tiles * S < cus && a.nbatch == 1 && S < 8 && a.K % (64 * 2 * S) == 0 &&
          a.K / (2 * S) >= 1024)
     S *= 2;
   if (tiles * S < cus)

@@ -551,3 +551,32 @@ def test_split_product_has_no_mean_shift(gpu, dist, K_):
     # rows' largest; independent ones: 4.5 of their standard deviations
     per = np.sqrt(K_ / 32 + 2) * 2.0**-24 * np.abs(want).max() / np.sqrt(3 * 4096)
     assert np.abs(err.mean(0)).max() <= 4.5 * per
+
+
+@pytest.mark.parametrize("layout", ["NN", "TN"])
+@pytest.mark.parametrize("M,K_,N", [(1020, 8200, 4100), (2300, 4101, 2305), (2048, 8192, 1024)])
+def test_split_product_fallback_is_the_fp32_product(gpu, M, K_, N, layout):
+    """A product whose data is outside the planes' range: bit for bit what the
+    fp32 kernels give it as a layer's forward (same tiles, same slices of K),
+    written, accumulated and with a bias, each added once; 16- and 4-byte
+    loads, and the split 256x256 tile."""
+    r = rng(seed_of("split-fallback", M, K_, N, layout))
+    a = r.standard_normal((M, K_), dtype=np.float32)
+    a[17, 5] = np.inf
+    xa = dev_T(a) if layout == "TN" else dev(a)
+    xb = dev(r.standard_normal((K_, N), dtype=np.float32))
+    bias = dev(r.standard_normal(N, dtype=np.float32))
+    old = r.standard_normal((M, N), dtype=np.float32)
+
+    def rows(x):
+        return np.delete(x, 17, 0)
+
+    def run(op, *args):
+        return rows(host(nt.Tensor._new_contiguous(op(*args, (M, N)), (M, N))))
+
+    want = run(K.linear, xa, xb, dev(np.zeros(N, np.float32)))
+    assert_bitexact(run(K.matmul, xa, xb), want, "written")
+    tgt = dev(old)
+    K.matmul_into(xa, xb, tgt, accumulate=True)
+    assert_bitexact(rows(host(tgt)), rows(old) + want, "accumulated")
+    assert_bitexact(run(K.matmul_bias, xa, xb, bias), run(K.linear, xa, xb, bias), "bias")
