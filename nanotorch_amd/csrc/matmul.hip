@@ -311,16 +311,20 @@ __device__ __forceinline__ void dl_wait_and_sync() {
   __syncthreads();
 }
 
-constexpr uint32_t SP_BAD = 1, SP_SMALL = 2;
-
-// Flags of both operands of a split product (mm_split_pack_kernel): whether
-// it is within the range where the parts do what float32 does.  SP_BAD: a
-// value that is not finite, 2^50 or more, or non-zero below 2^-60; SP_SMALL: a
-// non-zero one below 2^-40.  Without SP_BAD, and with SP_SMALL in at most one
-// operand, every non-zero product is in [2^-100, 2^100]: the products of its
-// parts, down to 2^-24 of it, are normal, and 2^27 of them cannot overflow.
-__device__ __forceinline__ bool split_ok(const uint32_t *flags) {
-  return !((flags[0] | flags[1]) & SP_BAD) && !(flags[0] & flags[1] & SP_SMALL);
+// Range of a split product (mm_split_pack_kernel).  flags[0], flags[1]: the
+// largest biased exponent in A and in B, or SP_HIGH if none is above.  Values
+// are packed times 2^SP_SHIFT, so that every part of every float32, subnormal
+// ones too, is a normal bfloat16, and what a product of parts loses below the
+// normal range is under 2^-170, past the last bit of any float32.  What is
+// left is the upper end: finite parts (values below 2^103), and K products
+// below 2^(ea + eb + 2) times 2^(2 SP_SHIFT) that cannot overflow.
+constexpr int SP_SHIFT = 24;
+constexpr uint32_t SP_HIGH = 127 + 10;
+__device__ __forceinline__ bool split_ok(const uint32_t *flags, int64_t K) {
+  const int bits = 64 - __builtin_clzll(uint64_t(K)); // K < 2^bits
+  const uint32_t ea = flags[0], eb = flags[1];
+  return ea < 127 + 103 && eb < 127 + 103 &&
+         int(ea + eb) - 2 * 127 + 2 + 2 * SP_SHIFT + bits <= 127;
 }
 
 // A BM x BN tile of a slice of K: 4 waves in a WM x WN grid, each a
@@ -350,7 +354,7 @@ void mm_f32_tile_kernel(MMArgs g) {
   const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wm = wave / WN, wn = wave % WN;
   const int h = lane >> 5, li = lane & 31;
-  if (g.flags && split_ok(g.flags) != g.run_if)
+  if (g.flags && split_ok(g.flags, g.K) != g.run_if)
     return;
   const TileCoord tc = mm_tile_coord<BM, BN>(g);
 
@@ -618,7 +622,7 @@ __global__ __launch_bounds__(WD_THREADS, 1) void mm_f32_mfma_wide_kernel(
   const int lane = t & 63, wave = t >> 6;
   const int wm = wave >> 2, wn = wave & 3;
   const int h = lane >> 5, li = lane & 31;
-  if (g.flags && split_ok(g.flags) != g.run_if)
+  if (g.flags && split_ok(g.flags, g.K) != g.run_if)
     return;
   const TileCoord tc = mm_tile_coord<WD_BM, WD_BN>(g);
 
@@ -708,12 +712,11 @@ __global__ __launch_bounds__(WD_THREADS, 1) void mm_f32_mfma_wide_kernel(
 // planes, in the order in which the product's LDS stages hold them, zeros
 // past every edge; mm_split_kernel multiplies; the slices of a split K are
 // added as for the other tiles.  What six exact products cannot do as the
-// fp32 kernel does -- infinities and NaN (0 x inf among the parts), parts or
-// products outside the normal range -- the pack kernel reports in a flag
-// word per operand: then mm_split_kernel returns at once and the fp32
-// kernel queued behind it does the work; otherwise that one returns at once.
-// (Out of range, 8192x4096x4096 takes 2059 us, 1974 without the packing; 4000^3
-// 1116 / 1071; 1024x8192x4096 685 / 581, whose K is not split then.)
+// fp32 kernel does -- infinities and NaN (0 x inf among the parts), values and
+// products near the upper end of float32's range -- the pack kernel reports
+// in a word per operand (split_ok): then it packs no further, mm_split_kernel
+// returns at once and the fp32 kernel queued behind it does the work;
+// otherwise that one returns at once.
 constexpr int SP_B = 256, SP_K = 16;             // rows of a block, k of a step
 constexpr int SP_PLANE = SP_B * SP_K;            // bf16 values
 constexpr int SP_STEP = 3 * SP_PLANE * 2;        // bytes of a block's k step
@@ -723,7 +726,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 __global__ void mm_split_flags_kernel(uint32_t *flags) {
   if (threadIdx.x < 2)
-    flags[threadIdx.x] = 0;
+    flags[threadIdx.x] = SP_HIGH;
 }
 
 struct SplitOperand {
@@ -752,6 +755,11 @@ __global__ __launch_bounds__(256) void mm_split_pack_kernel(
     return;
   const int64_t row = int64_t(rb) * 32 + lane % 32;
   const int64_t k = int64_t(step) * SP_K + lane / 32 * 8;
+  auto read = [&](int i) {
+    return uint32_t(__builtin_amdgcn_readfirstlane(
+        __hip_atomic_load(flags + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)));
+  };
+  const uint32_t seen[2] = {read(0), read(1)};
   float v[8];
   if (o.vec && row < o.rows && k + 8 <= K) {
     const float4 *q = reinterpret_cast<const float4 *>(o.p + row * o.s_mn + k);
@@ -766,16 +774,17 @@ __global__ __launch_bounds__(256) void mm_split_pack_kernel(
         v[e] = o.p[row * o.s_mn + (k + e) * o.s_k];
     }
   }
+  if (!split_ok(seen, K)) // another wave has settled it: nothing is packed
+    return;
   bf16x8 p1, p2, p3;
-  uint32_t f = 0;
+  uint32_t high = 0;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const uint32_t ex = (__float_as_uint(v[e]) >> 23) & 255; // 127: 1.x
-    const bool zero = v[e] == 0.f;
-    f |= ex >= 127 + 50 || (!zero && ex < 127 - 60) ? SP_BAD : 0;
-    f |= !zero && ex < 127 - 40 ? SP_SMALL : 0;
-    p1[e] = __bf16(v[e]);
-    const float r = v[e] - float(p1[e]);
+    high = high > ex ? high : ex;
+    const float x = v[e] * float(1 << SP_SHIFT);
+    p1[e] = __bf16(x);
+    const float r = x - float(p1[e]);
     p2[e] = __bf16(r);
     p3[e] = __bf16(r - float(p2[e]));
   }
@@ -784,8 +793,15 @@ __global__ __launch_bounds__(256) void mm_split_pack_kernel(
   *reinterpret_cast<bf16x8 *>(dst) = p1;
   *reinterpret_cast<bf16x8 *>(dst + 2 * SP_PLANE) = p2;
   *reinterpret_cast<bf16x8 *>(dst + 4 * SP_PLANE) = p3;
-  if (f) // rare: no traffic on the word for ordinary data
-    atomicOr(flags + second, f);
+  if (__any(high > seen[second])) { // no traffic on the word for ordinary data
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t other = __shfl_xor(high, off, 64);
+      high = high > other ? high : other;
+    }
+    if (lane == 0)
+      atomicMax(flags + second, high);
+  }
 }
 
 // 256x128 tiles, 8 waves in a 4x2 grid (two per SIMD) of 64x64: 2x2 blocks of
@@ -802,7 +818,7 @@ __global__ __launch_bounds__(256) void mm_split_pack_kernel(
 __global__ __launch_bounds__(512, 1) void mm_split_kernel(
     MMArgs g, const char *pa, const char *pb, uint32_t ksteps, uint32_t kper,
     const uint32_t *flags) {
-  if (!split_ok(flags))
+  if (!split_ok(flags, g.K))
     return;
   __shared__ __align__(16) char st0[SP_STAGE], st1[SP_STAGE], st2[SP_STAGE], st3[SP_STAGE];
   const int lane = threadIdx.x & 63;
@@ -947,7 +963,8 @@ __global__ __launch_bounds__(512, 1) void mm_split_kernel(
         const int64_t row =
             tc.m0 + wm * 64 + i * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
         if (row < g.M) // + 0: a sum of zeros is +0, as in the fp32 kernels
-          mm_put(g, tc, row, col, acc[i][j][r] + low[i][j][r] + 0.f);
+          mm_put(g, tc, row, col,
+                 (acc[i][j][r] + low[i][j][r]) * (1.f / (1ull << 2 * SP_SHIFT)) + 0.f);
       }
     }
 }
@@ -961,7 +978,7 @@ __global__ __launch_bounds__(256) void mm_splitk_sum_kernel(
   // one work-item per V columns of one row, in a one-shot grid; the S slice
   // loads are independent (S is a template argument) and go out together
   const uint32_t q = blockIdx.x * 256u + threadIdx.x;
-  if (q >= total || (g.flags && split_ok(g.flags) != g.run_if))
+  if (q >= total || (g.flags && split_ok(g.flags, g.K) != g.run_if))
     return;
   const uint32_t rm = fdn.div(q); // batch * M + m
   const int64_t n = int64_t(q - rm * fdn.d) * V;

@@ -580,3 +580,38 @@ def test_split_product_fallback_is_the_fp32_product(gpu, M, K_, N, layout):
     K.matmul_into(xa, xb, tgt, accumulate=True)
     assert_bitexact(rows(host(tgt)), rows(old) + want, "accumulated")
     assert_bitexact(run(K.matmul_bias, xa, xb, bias), run(K.linear, xa, xb, bias), "bias")
+
+
+@pytest.mark.parametrize("values", ["one tiny", "softmax", "subnormal rows", "far apart"])
+def test_split_product_of_wide_ranges(gpu, values):
+    """Values down to the subnormals, and operands of very different size,
+    stay on the planes (other last bits than the fp32 kernels): less than half
+    of the fp32 kernels' error in 2-norm, and each result within the bound of
+    a float32 sum (plus the spacing of the subnormals where it is one).  Of
+    the softmax-like rows, exp(12 n - 50), one term is nearly all of the
+    2-norm: there it is one rounding and the products left out against one
+    rounding, rms 0.436 against 0.425 of 2^-24."""
+    M, K_, N = 4096, 320, 4096
+    r = rng(seed_of("split-wide", values))
+    a = r.standard_normal((M, K_), dtype=np.float32)
+    b = r.standard_normal((K_, N), dtype=np.float32)
+    if values == "one tiny":
+        a[17, 5] = 2.0**-70
+    elif values == "softmax":
+        a = np.exp(12 * a - 50) / np.float32(8192)  # 2^-126 and below to about 1
+    elif values == "subnormal rows":
+        a[17] *= np.float32(2.0**-130)
+        a[18] *= np.float32(2.0**-110)
+    else:
+        a *= np.float32(2.0**50)
+        b *= np.float32(2.0**-60)
+    xa, xb = dev(a), dev(b)
+    got = _mm(xa, xb)
+    zero = dev(np.zeros(N, np.float32))
+    fp32 = host(nt.Tensor._new_contiguous(K.linear(xa, xb, zero, (M, N)), (M, N)))
+    want = a.astype(np.float64) @ b
+    scale = np.abs(a).astype(np.float64) @ np.abs(b)
+    assert (np.abs(got - want) <= K_ * 2.0**-24 * scale + 2.0**-149).all()
+    assert (got != fp32).any()
+    most = 1.05 if values == "softmax" else 0.5
+    assert np.linalg.norm(got - want) < most * np.linalg.norm(fp32 - want)
