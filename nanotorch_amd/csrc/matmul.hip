@@ -170,7 +170,9 @@ enum { ST_K16 = 0, ST_MN16 = 1, ST_K4 = 2, ST_MN4 = 3 };
 // collide: rocprof counted one LDS bank conflict per read.)
 __device__ __forceinline__ int dl_swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
-template <int ST, int B> struct StageTile {
+// FAR: strides past the 32-bit offsets (64 rows of 2^22 elements and more):
+// a 64-bit offset per load.
+template <int ST, int B, bool FAR = false> struct StageTile {
   static constexpr int FLOATS = ST == ST_K4 ? B / 2 * 68 : B * MM_BK;
   static constexpr bool WIDE = ST == ST_K16 || ST == ST_MN16;
   static constexpr int NI = WIDE ? B / 32 : B / 8; // instructions per wave
@@ -184,8 +186,9 @@ template <int ST, int B> struct StageTile {
     else
       return k * B + mn;
   }
+  using Off = std::conditional_t<FAR, int64_t, uint32_t>;
   const char *base;  // element (mn0, k0) of the operand
-  uint32_t off[NI];  // byte offset of this lane's source, instruction j
+  Off off[NI];       // byte offset of this lane's source, instruction j
   int64_t kstep;     // bytes between two k-tiles
   __device__ __forceinline__ void init(const float *p, int64_t mn0, int64_t MN,
                                        int64_t s_mn, int64_t s_k, int wave,
@@ -195,7 +198,7 @@ template <int ST, int B> struct StageTile {
     // the last row (16-byte group of rows) that may be read
     const int64_t last = MN - mn0 - (ST == ST_MN16 ? 4 : 1);
     const int lastc = int(last < B - 1 ? last : B - 1);
-    const uint32_t bm = uint32_t(4 * s_mn), bk = uint32_t(4 * s_k);
+    const Off bm = Off(4 * s_mn), bk = Off(4 * s_k);
 #pragma unroll
     for (int j = 0; j < NI; ++j) {
       const int q = wave * NI + j;
@@ -216,11 +219,25 @@ template <int ST, int B> struct StageTile {
         mn = flat % B;
       }
       mn = mn < lastc ? mn : lastc;
-      off[j] = uint32_t(mn) * bm + uint32_t(k) * bk;
+      off[j] = Off(mn) * bm + Off(k) * bk;
     }
   }
   __device__ __forceinline__ void issue(float *stage, int64_t kt,
                                         int wave) const {
+    if constexpr (FAR) {
+#pragma unroll
+      for (int j = 0; j < NI; ++j) {
+        auto *from =
+            (const __attribute__((address_space(1))) void *)(base + kt * kstep + off[j]);
+        auto *to = (__attribute__((address_space(3))) void *)(stage +
+                                                              (wave * NI + j) * LDS_STEP);
+        if constexpr (WIDE)
+          __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
+        else
+          __builtin_amdgcn_global_load_lds(from, to, 4, 0, 0);
+      }
+      return;
+    }
     // Buffer loads: a scalar base and each lane's 32-bit offset.  (With
     // global pointers the compiler kept a 64-bit address per load in
     // registers and advanced them all each k-tile, and spilled in the
@@ -341,11 +358,11 @@ __device__ __forceinline__ bool split_ok(const uint32_t *flags, int64_t K) {
 // four times the load instructions of the 16-byte ones and run at 0.8 of
 // their rate; through registers, one strided element at a time, odd row
 // lengths had run at a fifth of it.
-template <int SA, int SB, int BM, int BN>
+template <int SA, int SB, int BM, int BN, bool FAR = false>
 __global__ __launch_bounds__(MM_THREADS, BM * BN >= 128 * 128 ? 2 : 3)
 void mm_f32_tile_kernel(MMArgs g) {
-  using TA = StageTile<SA, BM>;
-  using TB = StageTile<SB, BN>;
+  using TA = StageTile<SA, BM, FAR>;
+  using TB = StageTile<SB, BN, FAR>;
   constexpr int WN = BM == BN ? 2 : (BM < BN ? 4 : 1), WM = 4 / WN;
   constexpr int NM = BM / WM / 32, NN = BN / WN / 32;
   __shared__ __align__(16) float sA0[TA::FLOATS], sB0[TB::FLOATS];
@@ -431,78 +448,6 @@ void mm_f32_tile_kernel(MMArgs g) {
       for (int r = 0; r < 16; ++r) {
         const int64_t row =
             tc.m0 + wm * (BM / WM) + i * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
-        if (row < g.M)
-          mm_put(g, tc, row, col, acc[i][j][r]);
-      }
-    }
-}
-
-// Any strides at all (64-bit offsets, through registers): operands whose
-// strides exceed the tile kernel's 32-bit offsets (a row stride past 2^22
-// elements), 128x128 tiles.
-__global__ __launch_bounds__(MM_THREADS, 2) void mm_f32_far_kernel(MMArgs g) {
-  constexpr int P = MM_BK + 4; // padded [mn][k] row
-  __shared__ __align__(16) float lds[2][128 * P];
-  const int t = threadIdx.x;
-  const int lane = t & 63, wave = t >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int h = lane >> 5, li = lane & 31;
-  const TileCoord tc = mm_tile_coord<128, 128>(g);
-  floatx16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        acc[i][j][r] = 0.f;
-  for (int64_t k0 = 0; k0 < g.K; k0 += MM_BK) {
-    float va[16], vb[16];
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int flat = t + MM_THREADS * e;
-      const int64_t mn = flat >> 5, k = k0 + (flat & 31);
-      va[e] = vb[e] = 0.f;
-      if (tc.m0 + mn < g.M && k < g.K)
-        va[e] = tc.A[(tc.m0 + mn) * g.sAm + k * g.sAk];
-      if (tc.n0 + mn < g.N && k < g.K)
-        vb[e] = tc.B[(tc.n0 + mn) * g.sBn + k * g.sBk];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int flat = t + MM_THREADS * e;
-      lds[0][(flat >> 5) * P + (flat & 31)] = va[e];
-      lds[1][(flat >> 5) * P + (flat & 31)] = vb[e];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      float a[2], b[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        a[i] = lds[0][(wm * 64 + i * 32 + li) * P + h * 16 + kk];
-        b[i] = lds[1][(wn * 64 + i * 32 + li) * P + h * 16 + kk];
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j],
-                                                           acc[i][j], 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int64_t col = tc.n0 + wn * 64 + j * 32 + li;
-      if (col >= g.N)
-        continue;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t row =
-            tc.m0 + wm * 64 + i * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
         if (row < g.M)
           mm_put(g, tc, row, col, acc[i][j][r]);
       }
@@ -1267,7 +1212,7 @@ struct TileChoice {
   double us; // the estimate
 };
 
-TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int64_t nbatch) {
+TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int64_t nbatch, bool only64 = false) {
   constexpr double TK128 = 2.3, TK = 1.8; // us per 128x128x32 of MFMAs on a CU
   constexpr double LAT128 = 0.65, LAT = 0.49, EPI = 1.07;
   constexpr double SUM = 2.2, SUM_BYTES = 8.8e6; // us, bytes per us
@@ -1290,6 +1235,8 @@ TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int64_t nbatch) {
   double best_t = std::numeric_limits<double>::infinity();
   for (const auto &sh : SHAPES) {
     const int bm = sh[0], bn = sh[1];
+    if (only64 && (bm != 64 || bn != 64))
+      continue;
     const bool big = bm == 128 && bn == 128;
     const double area = bm * bn / (128. * 128.);
     const int64_t tiles = ceil_div(M, bm) * ceil_div(N, bn) * nbatch;
@@ -1311,7 +1258,7 @@ TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int64_t nbatch) {
   return best;
 }
 
-template <int SA, int SB, int BM, int BN>
+template <int SA, int SB, int BM, int BN, bool FAR = false>
 void launch_tile(const MMArgs &a, const TileChoice &c) {
   run_split(a, c.S, c.kslice, [](MMArgs w, int S) {
     w.tiles_m = ceil_div(w.M, BM);
@@ -1319,12 +1266,17 @@ void launch_tile(const MMArgs &a, const TileChoice &c) {
     const int64_t blocks = w.tiles_m * w.tiles_n * w.nbatch * S;
     if (blocks >= (int64_t(1) << 31))
       fail(NT_ERR_RUNTIME, "matmul: problem too large");
-    mm_f32_tile_kernel<SA, SB, BM, BN>
+    mm_f32_tile_kernel<SA, SB, BM, BN, FAR>
         <<<dim3(unsigned(blocks)), MM_THREADS, 0, stream()>>>(w);
   });
 }
 
-template <int SA, int SB> void launch_stages(const MMArgs &a) {
+template <int SA, int SB> void launch_stages(const MMArgs &a, bool far) {
+  // Far strides: 64x64 only (64-bit offsets of a 128x128 tile's stages would
+  // spill).  [64, 8M] times its transpose 743 ms (one element at a time through
+  // registers, K unsplit) -> 17, its transpose times [64, 64] 3.2 -> 1.2.
+  if (far)
+    return launch_tile<SA, SB, 64, 64, true>(a, choose_tile(a.M, a.N, a.K, a.nbatch, true));
   const TileChoice c = choose_tile(a.M, a.N, a.K, a.nbatch);
   if (c.bm == 64)
     launch_tile<SA, SB, 64, 64>(a, c);
@@ -1476,14 +1428,14 @@ void launch_f32(const MMArgs &a, bool al, bool planes) {
   auto tiles = [&](const MMArgs &g) {
     if (wide) {
       if (a_mn)
-        b_mn ? launch_stages<ST_MN16, ST_MN16>(g) : launch_stages<ST_MN16, ST_K16>(g);
+        b_mn ? launch_stages<ST_MN16, ST_MN16>(g, far) : launch_stages<ST_MN16, ST_K16>(g, far);
       else
-        b_mn ? launch_stages<ST_K16, ST_MN16>(g) : launch_stages<ST_K16, ST_K16>(g);
+        b_mn ? launch_stages<ST_K16, ST_MN16>(g, far) : launch_stages<ST_K16, ST_K16>(g, far);
     } else {
       if (a_mn)
-        b_mn ? launch_stages<ST_MN4, ST_MN4>(g) : launch_stages<ST_MN4, ST_K4>(g);
+        b_mn ? launch_stages<ST_MN4, ST_MN4>(g, far) : launch_stages<ST_MN4, ST_K4>(g, far);
       else
-        b_mn ? launch_stages<ST_K4, ST_MN4>(g) : launch_stages<ST_K4, ST_K4>(g);
+        b_mn ? launch_stages<ST_K4, ST_MN4>(g, far) : launch_stages<ST_K4, ST_K4>(g, far);
     }
   };
   auto large = [&](const MMArgs &g) {
@@ -1508,17 +1460,6 @@ void launch_f32(const MMArgs &a, bool al, bool planes) {
   }
   if (large(a))
     return;
-  if (far) {
-    MMArgs w = a;
-    w.kslice = a.K;
-    w.tiles_m = ceil_div(a.M, 128);
-    w.tiles_n = ceil_div(a.N, 128);
-    const int64_t blocks = w.tiles_m * w.tiles_n * w.nbatch;
-    if (blocks >= (int64_t(1) << 31))
-      fail(NT_ERR_RUNTIME, "matmul: problem too large");
-    mm_f32_far_kernel<<<dim3(unsigned(blocks)), MM_THREADS, 0, stream()>>>(w);
-    return;
-  }
   tiles(a);
 }
 

@@ -615,3 +615,42 @@ def test_split_product_of_wide_ranges(gpu, values):
     assert (got != fp32).any()
     most = 1.05 if values == "softmax" else 0.5
     assert np.linalg.norm(got - want) < most * np.linalg.norm(fp32 - want)
+
+
+@pytest.mark.parametrize("K_", [68, 71, 2100])  # 16- and 4-byte loads, a tail, K split
+@pytest.mark.parametrize("form", ["A", "A.T", "B", "B.T", "both"])
+def test_far_strides(gpu, form, K_):
+    """Operands whose rows (or, transposed, whose k's) lie over 2^22 elements
+    apart, beside one of ordinary strides or another such; 70 rows are two
+    tiles, the second ragged.  Every output against the fp64 product, written
+    and accumulated."""
+    r = rng(seed_of("far", form, K_))
+    rows, off = 72 if form.endswith("T") else 70, 4 if K_ % 4 == 0 else 3
+    big = nt.zeros(rows, 2**22 + 2200, device="cuda")
+    n = 44  # columns of a transposed far operand
+    vals = r.standard_normal((rows, n if form.endswith("T") else K_), dtype=np.float32)
+    big[:, off:off + vals.shape[1]] = dev(vals)
+    far = big[:, off:off + vals.shape[1]]
+    if form == "A":  # [rows, K] . [K, n]
+        b = r.standard_normal((K_, n), dtype=np.float32)
+        xa, xb, a = far, dev(b), vals
+    elif form == "B.T":  # [n, rows] . [rows, n]: k walks the far rows of B
+        a = r.standard_normal((52, rows), dtype=np.float32)
+        xa, xb, b = dev(a), far, vals
+    elif form == "A.T":
+        b = r.standard_normal((rows, 52), dtype=np.float32)
+        xa, xb, a = far.T, dev(b), vals.T
+    elif form == "B":  # [52, K] . [K, rows], B column-major
+        a = r.standard_normal((52, K_), dtype=np.float32)
+        xa, xb, b = dev(a), far.T, vals.T
+    else:
+        xa, xb, a, b = far, far.T, vals, vals.T
+    want = a.astype(np.float64) @ b
+    scale = np.abs(a).astype(np.float64) @ np.abs(b)
+    old = r.standard_normal(want.shape, dtype=np.float32)
+    tgt = dev(old)
+    for acc in (False, True):
+        K.matmul_into(xa, xb, tgt, accumulate=acc)
+        # K products in any order, the slices' sums and the accumulate
+        bound = 2 * (a.shape[1] + 2) * 2.0**-24 * scale * (2 if acc else 1)
+        assert (np.abs(host(tgt) - want * (2 if acc else 1)) <= bound).all()
