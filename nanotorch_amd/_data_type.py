@@ -44,7 +44,7 @@ def ctype_of(dtype: Dtype):
 
 def sizeof(dtype: Dtype) -> int:
     """Bytes per element (reference: core.py:35-44)."""
-    return _SIZES[dtype]
+    return _SIZES[dtype if type(dtype) is Dtype else Dtype(dtype)]
 
 
 def dtype_from_type(data: InputType) -> Dtype:

@@ -45,3 +45,12 @@ def test_reshape_view_refuses_another_size():
     for dims in ((2, 4), (5,), (), (0,), (13,)):
         with pytest.raises(ValueError):
             reshape_view(x, dims)
+
+
+def test_sizeof_refuses_an_unknown_dtype():
+    from nanotorch_amd._data_type import Dtype, sizeof
+
+    assert [sizeof(d) for d in Dtype] == [sizeof(int(d)) for d in Dtype] == [1, 4, 8, 4, 8]
+    for bad in (17, "float32", None, []):
+        with pytest.raises(ValueError):
+            sizeof(bad)
