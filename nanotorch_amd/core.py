@@ -684,7 +684,7 @@ def _run_backward(fn, grad: Tensor, inputs: tuple) -> None:
             sub_needs = needs if grp is None else [
                 needs[i] and i in grp for i in range(len(inputs))
             ]
-            if True not in sub_needs:
+            if not any(sub_needs):
                 continue
             targets = [
                 _accumulation_target(x) if n else None

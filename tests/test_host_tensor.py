@@ -54,3 +54,25 @@ def test_sizeof_refuses_an_unknown_dtype():
     for bad in (17, "float32", None, []):
         with pytest.raises(ValueError):
             sizeof(bad)
+
+
+def test_any_true_requires_grad_gets_its_gradient():
+    """requires_grad is taken by its truth (the constructor keeps what it was
+    given), in the fused backward as everywhere else."""
+    from nanotorch_amd.autograd.function import Function
+    from nanotorch_amd.core import _run_backward
+
+    class Twice(Function):
+        def fused_ok(self):
+            return True
+
+        def _backward_into(self, g, needs, targets):
+            return [nt.Tensor([2 * v for v in g.tolist()]) if n else None for n in needs]
+
+    for flag in (True, 1, 2, "yes"):
+        x = nt.Tensor([1.0], requires_grad=flag)
+        _run_backward(Twice(), nt.Tensor([3.0]), (x,))
+        assert x.grad is not None and x.grad.tolist() == [6.0], flag
+    x = nt.Tensor([1.0])
+    _run_backward(Twice(), nt.Tensor([3.0]), (x,))
+    assert x.grad is None
