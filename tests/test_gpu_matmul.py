@@ -184,8 +184,10 @@ def test_wide_tile_split_k_full_check(gpu, accumulate, layout):
 
 BIAS_SHAPES = [(7, 5, 3), (129, 33, 130), (300, 257, 512),  # generic / edge tiles
                (1024, 512, 768),                            # 128x128 MFMA kernels
-               (4096, 1024, 4096),                          # wide kernel, one pass
-               (1024, 8192, 256),                           # wide kernel, split K
+               (4096, 1024, 4096),                          # bf16 planes, one slice
+               (1024, 8192, 4100),                          # bf16 planes, split K
+               (4096, 64, 4096),                            # wide kernel, one pass
+               (1024, 8192, 256),                           # tile kernels, split K
                (64, 0, 96)]                                  # K = 0: C = bias
 
 

@@ -293,6 +293,12 @@ def test_split_slices_back_to_back(gpu):
     ((1 << 20,), (0,)),       # full reduction
     ((4096, 1030), (0,)),     # column walk (wide blocks and a ragged edge)
     ((37, 9, 401), (0, 2)),   # generic kernel
+    # short rows: 4, 16 and 64 lanes a slice, 4- and 16-byte loads
+    ((70, 5), (1,)), ((70, 16), (1,)), ((70, 32), (1,)), ((70, 33), (1,)), ((70, 130), (1,)),
+    ((70, 256), (1,)), ((1001, 2051), (1,)), ((1001, 4092), (1,)), ((64, 7, 6), (2,)),
+    # column walk: 4, 16 and 64 lanes, split or not, batched, ragged edges
+    ((5000, 7), (0,)), ((5000, 40), (0,)), ((5000, 132), (0,)), ((9, 5, 15), (1,)),
+    ((9, 197, 64), (1,)), ((9, 197, 1030), (1,)), ((8, 3000, 33), (1,)),
 ])
 def test_select_special_values(gpu, shape, axes):
     """Max / min / argmax / argmin and tie counts over +-inf, the neutral
@@ -435,3 +441,26 @@ def test_broadcast_over_a_middle_axis(gpu, C, dt):
     t[:, 2] = dev(a) * dev(m).to(nt.float64 if dt == "f64" else nt.float32)
     big[:, 2] = a * m
     assert_bitexact(host(t), big, "sliced output")
+
+
+@pytest.mark.parametrize("shape,axis", [
+    ((70, 5), 1), ((70, 33), 1), ((70, 130), 1), ((1001, 2051), 1), ((1001, 4092), 1),
+    ((5000, 7), 0), ((5000, 40), 0), ((9, 197, 64), 1), ((9, 197, 1030), 1), ((8, 3000, 33), 1)])
+def test_sum_special_values_stay_in_their_slice(gpu, shape, axis):
+    """Infinities and NaN among small integers, the last elements of a slice
+    (which short rows load again to fill a group) included: the slices that
+    hold them sum to what they must, every other one exactly."""
+    r = rng(seed_of("sum-special", shape, axis))
+    a = r.integers(-9, 10, shape).astype(np.float32)
+    flat = np.moveaxis(a, axis, 0)  # a view: [reduced, kept...]
+    kept = [(i,) * (a.ndim - 1) for i in range(5)]
+    flat[(-1,) + kept[0]] = np.inf
+    flat[(0,) + kept[1]] = -np.inf
+    flat[(-1,) + kept[2]] = np.nan
+    flat[(0,) + kept[3]], flat[(-1,) + kept[3]] = np.inf, -np.inf
+    flat[(-2,) + kept[4]] = np.inf
+    with np.errstate(invalid="ignore"):
+        want = a.sum(axis=axis)
+    got = host(dev(a).sum(axis))
+    assert_bitexact(np.isnan(got), np.isnan(want), "NaN")
+    assert (got[~np.isnan(want)] == want[~np.isnan(want)]).all()
