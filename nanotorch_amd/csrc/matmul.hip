@@ -755,11 +755,11 @@ __global__ __launch_bounds__(256) void mm_split_pack_kernel(
 // reads (half of the LDS rate), so the matrix pipe and the chip's power (the
 // clock falls below 2 GHz) are the bound.  Stages are copies of the packed
 // operands (every load 1 KB of consecutive memory, conflict-free reads).
-// With packing, in us, fp32 MFMA -> this: 8192x4096x4096 1980 -> 1393,
-// 4000^3 1075 -> 738, 1024x8192x4096 510 -> 420, 8192x4096x1000 520 -> 398,
-// 4096x300x4096 109 -> 81.  (One running sum of all six products in 256x256
-// tiles, every sum rounded down: 4000^3 682 us, with five times the error; the
-// leading products of each step added apart: 759.)
+// With packing, in us, fp32 MFMA -> this: 8192x4096x4096 1949 -> 1345,
+// 4000^3 1074 -> 708, 1024x8192x4096 511 -> 408, 8192x4096x1000 518 -> 387,
+// 4093x301x4090 112 -> 84.  (Where this takes 738 for 4000^3: one running sum
+// of all six products in 256x256 tiles, every sum rounded down, 682, with five
+// times the error; the leading products of each step added apart, 759.)
 __global__ __launch_bounds__(512, 1) void mm_split_kernel(
     MMArgs g, const char *pa, const char *pb, uint32_t ksteps, uint32_t kper,
     const uint32_t *flags) {
@@ -1329,14 +1329,15 @@ template <int LA, int LB> bool launch_wide(const MMArgs &a) {
 }
 
 // The product through packed bf16 planes (mm_split_kernel), where that is
-// estimated to take no longer than the fp32 kernels' f32_us (an estimate too,
-// of 0.8 to 1 of what they measured); false: not taken.  A k step of a tile
-// takes 0.8 us with few CUs at work and 1.12 with all (the clock falls with
-// the power), packing 10 bytes per value at 5 TB/s and the three small
-// launches 12 us; measured / estimated / fp32 measured, in us: 4000^3 665 /
-// 660 / 1050, 8192x4096x1000 388 / 383 / 572, 1024x8192x4096 410 / 404 / 556,
-// 2912x2804x6472 625 / 646 / 900, 4093x301x4090 80 / 80 / 118.  ak, bk: the
-// operand has 16-byte aligned rows along k.
+// estimated to take no longer than the fp32 kernels, f32_us; false: not taken.
+// A k step of a tile takes 0.8 us with few CUs at work and 1.12 with all (the
+// clock falls with the power), packing 10 bytes per value at 5 TB/s and the
+// three small launches 12 us; measured / estimated / fp32 measured, in us:
+// 4000^3 630 / 660 / 1021, 8192x4096x1000 367 / 383 / 529, 1024x8192x4096
+// 401 / 404 / 505, 6112x868x3912 229 / 245 / 365, 4096x320x4096 78 / 80 / 101.
+// Over 32 products that take the planes they were 1.13 to 1.70 times as fast as
+// the fp32 kernels, 1.34 in the mean.  ak, bk: the operand has 16-byte aligned
+// rows along k.
 template <class FB>
 bool launch_split(const MMArgs &a, double f32_us, bool ak, bool bk, FB fallback) {
   if (f32_us < 40 || a.K >= (int64_t(1) << 27))
@@ -1445,16 +1446,16 @@ void launch_f32(const MMArgs &a, bool al, bool planes) {
                                  : launch_wide<LAY_K, LAY_K>(g)));
   };
   if (planes && !far && a.nbatch == 1) {
-    // large tiles at 131 TFLOP/s, or the tile kernel's estimate (4-byte loads
-    // at 0.8 of its rate)
+    // What the fp32 kernels take: large tiles at 131 TFLOP/s or the tile
+    // kernel's estimate, of which 0.96 to 1.5 were measured (4-byte loads:
+    // 1.09 to 1.3; medians 1.1 and 1.2 over 100 products).
     const double flops_us = 2. * double(a.M) * double(a.N) * double(a.K) / 131e6;
     if (flops_us > 20) {
-      const double est = choose_tile(a.M, a.N, a.K, 1).us;
-      if (launch_split(a, wide ? std::max(flops_us, est) : 1.25 * std::max(flops_us, est),
-                       ak, bk, [&](const MMArgs &g) {
-                         if (!large(g))
-                           tiles(g);
-                       }))
+      const double us = std::max(flops_us, choose_tile(a.M, a.N, a.K, 1).us);
+      if (launch_split(a, (wide ? 1.08 : 1.15) * us, ak, bk, [&](const MMArgs &g) {
+            if (!large(g))
+              tiles(g);
+          }))
         return;
     }
   }
