@@ -287,7 +287,8 @@ int nt_reduce_bwd(int32_t op, const nt_view *g, double scale, const nt_view *idx
  * dims arrive as stride-0 views).  Operand orientation is read from the
  * strides, so the backward products dA = dG.B^T and dB = A^T.dG
  * (src/nanotorch/autograd/ops_binary.py:253-267) are this call on transposed
- * views, read in place.  fp32 runs on the gfx950 fp32 MFMA units.  With
+ * views, read in place.  fp32 runs on the gfx950 fp32 MFMA units; large single
+ * products on the bf16 ones, each value split into three exact parts.  With
  * accumulate != 0, c = c_old + (a.b), one rounding after the full sum. */
 int nt_matmul(const nt_view *a, const nt_view *b, const nt_view *c,
               int32_t accumulate);
